@@ -1556,7 +1556,13 @@ void ensure_rows(SessionImpl& S, int rows) {
     S.att_part.alloc((size_t)rows * c.heads * S.max_splits * (c.head_dim + 2) * 4);
     S.att_arrived.alloc((size_t)rows * c.kv_heads * 4);
     const int kmax = std::max(std::max(c.d, qd), c.ffn);
-    S.gemm_scratch.alloc(std::max(gemm_scratch_bytes(rows, kmax), gemv_scratch_bytes(8, kmax)));
+    size_t scratch = std::max(gemm_scratch_bytes(rows, kmax), gemv_scratch_bytes(8, kmax));
+    // Float-math linears of many rows: their operand copy.
+    const DecoderImpl& D = *S.dec;
+    for (int l = 0; l < c.layers && rows > 8; ++l)
+        for (const Layer* L : {D.qkv[l].get(), D.o[l].get(), D.gate_up[l].get(), D.down[l].get()})
+            if (float_kind(L->kind)) scratch = std::max(scratch, gemm_float_scratch_want(rows, L->k));
+    S.gemm_scratch.alloc(scratch);
     TRIT_HIP(hipMemset(S.att_arrived.ptr, 0, (size_t)rows * c.kv_heads * 4));
     S.rows_cap = rows;
     drop_graph(S);
@@ -1580,6 +1586,8 @@ bool use_flash() {
 void product(SessionImpl& S, const Layer& L, GemvArgs a, int rows, hipStream_t s, int y_stride) {
     a.m = rows;
     if (rows > 8 && gemm_supported(L, a)) return gemm_int(L, a, S.gemm_scratch.ptr, s);
+    if (rows > 8 && gemm_float_mfma_supported(L, a))
+        return gemm_float_mfma(L, a, S.gemm_scratch.ptr, S.gemm_scratch.bytes, s);
     a.scratch = S.gemm_scratch.ptr;
     a.scratch_bytes = S.gemm_scratch.bytes;
     for (int r0 = 0; r0 < rows; r0 += 8) {

@@ -174,6 +174,28 @@ __device__ __forceinline__ float row_bcast(float v, int n) {
     }
 }
 
+// The 4 x 4 transpose between a lane's four registers and the wave's four
+// quarters (16 lanes each): v[j] in quarter q becomes what v[q] was in
+// quarter j, lane by lane of the quarter. The 32-lane swap exchanges the
+// high bits of j and q, the 16-lane swap the low bits.
+__device__ __forceinline__ void transpose_quarters(float (&v)[4]) {
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    auto bits = [](float f) { return __builtin_bit_cast(unsigned int, f); };
+    auto real = [](unsigned int u) { return __builtin_bit_cast(float, u); };
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const u32x2 r = __builtin_amdgcn_permlane32_swap(bits(v[j]), bits(v[j + 2]), false, false);
+        v[j] = real(r.x);
+        v[j + 2] = real(r.y);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j += 2) {
+        const u32x2 r = __builtin_amdgcn_permlane16_swap(bits(v[j]), bits(v[j + 1]), false, false);
+        v[j] = real(r.x);
+        v[j + 1] = real(r.y);
+    }
+}
+
 __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
     return __builtin_amdgcn_sdot4((int)a, (int)b, c, false);
 }

@@ -225,6 +225,11 @@ void encoder_product(const Layer& L, const float* x, int m, float* y, const floa
         return gemm_int(L, a, scratch.ptr, s);
     }
     if (m > 8 && gemm_float_supported(L, a)) return gemm_float(L, a, s);
+    if (m > 8 && gemm_float_mfma_supported(L, a)) {
+        const size_t need = gemm_float_scratch_want(m, L.k);
+        if (scratch.bytes < need) scratch.alloc(need);
+        return gemm_float_mfma(L, a, scratch.ptr, scratch.bytes, s);
+    }
     if (!float_kind(L.kind)) {
         const size_t need = gemv_scratch_bytes(8, L.k);
         if (scratch.bytes < need) scratch.alloc(need);

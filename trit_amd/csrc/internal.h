@@ -193,6 +193,18 @@ void gemv_float(const Layer& L, const GemvArgs& a, hipStream_t s);
 // SwiGLU pair): the same bits row by row.
 bool gemm_float_supported(const Layer& L, const GemvArgs& a);
 void gemm_float(const Layer& L, const GemvArgs& a, hipStream_t s);
+// Float-math products of any row count and k on the f32 matrix cores (no
+// prologue, no SwiGLU pair): the same bits. `scratch` is device memory the
+// product may overwrite: gemm_float_scratch_bytes(m, k) take all rows in
+// one pass, less takes passes of as many rows as fit (at least 16, or it
+// fails). gemm_float_scratch_want: what to give it, the whole up to 64 MiB.
+bool gemm_float_mfma_supported(const Layer& L, const GemvArgs& a);
+size_t gemm_float_scratch_bytes(int m, int k);
+inline size_t gemm_float_scratch_want(int m, int k) {
+    const size_t cap = (size_t)64 << 20, all = gemm_float_scratch_bytes(m, k), least = gemm_float_scratch_bytes(1, k);
+    return all < cap ? all : least > cap ? least : cap;
+}
+void gemm_float_mfma(const Layer& L, GemvArgs a, void* scratch, size_t scratch_bytes, hipStream_t s);
 // Integer products of any row count on the matrix cores (Q8_0, Q4_K, INT8;
 // k a multiple of the weight group, any n; the SwiGLU pair needs n / 2 a
 // multiple of 64). `scratch` holds gemm_scratch_bytes(m, k) bytes of

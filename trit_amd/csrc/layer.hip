@@ -1,5 +1,6 @@
 // The layer half of the C ABI (include/trit_hip.h): construction of the
 // device weight cache for each weight kind, and the products.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -325,16 +326,34 @@ void* staging_scratch(size_t need) {
     return g.scratch.ptr;
 }
 
+// The scratch bytes a product queued on `s` may ask of staging_scratch
+// beyond what it cannot do without: none while `s` is being captured (a
+// growth would allocate, and the graph would keep the old address).
+size_t staging_spare(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return status == hipStreamCaptureStatusNone ? SIZE_MAX : 0;
+}
+
 // One product of m rows: the matrix-core product for many rows, else the
 // small-batch kernels in calls of up to 8 rows (2..8 rows of an integer
 // layer with their activations quantized once, in the scratch). `get`
 // gives the scratch of `need` bytes (staging_scratch, or the no-allocation
-// array).
+// array). Products that take any amount of scratch get `spare` bytes at
+// most; 0: they run in the calls of up to 8 rows.
 template <class Scratch>
-void forward_rows(const Layer& L, GemvArgs a, int m, hipStream_t s, Scratch get) {
+void forward_rows(const Layer& L, GemvArgs a, int m, hipStream_t s, Scratch get, size_t spare) {
     a.m = m;
     if (m >= GEMM_MIN_ROWS && gemm_supported(L, a)) return gemm_int(L, a, get(gemm_scratch_bytes(m, L.k)), s);
     if (m > 8 && !a.ev_start && !a.ev_stop && gemm_float_supported(L, a)) return gemm_float(L, a, s);
+    if (m > 8 && !a.ev_start && !a.ev_stop && gemm_float_mfma_supported(L, a) &&
+        gemm_float_scratch_bytes(1, L.k) <= spare) {
+        const size_t bytes = std::min(spare, gemm_float_scratch_want(m, L.k));
+        return gemm_float_mfma(L, a, get(bytes), bytes, s);
+    }
     if (m >= 2 && !float_kind(L.kind)) {
         a.scratch_bytes = gemv_scratch_bytes(m < 8 ? m : 8, L.k);
         a.scratch = get(a.scratch_bytes);
@@ -694,7 +713,8 @@ int trit_hip_layer_forward_device(const TritHipLayer* layer, const float* x, int
         a.y = y;
         a.relu = relu;
         if (m <= 0) fail("m must be positive");
-        forward_rows(*layer->layer, a, m, s ? (hipStream_t)s : stream(), staging_scratch);
+        const hipStream_t st = s ? (hipStream_t)s : stream();
+        forward_rows(*layer->layer, a, m, st, staging_scratch, m > 8 ? staging_spare(st) : 0);
         return 0;
     });
 }
@@ -725,7 +745,7 @@ int trit_hip_layer_forward_device_noalloc(const TritHipLayer* layer, const float
                      std::to_string(L.k) + " layer need " + std::to_string(need) + " bytes of scratch, more than the " +
                      std::to_string(NOALLOC_SCRATCH_BYTES) + " it holds");
             return base;
-        });
+        }, NOALLOC_SCRATCH_BYTES);
         return 0;
     });
 }
@@ -741,7 +761,8 @@ int trit_hip_layer_forward_timed(const TritHipLayer* layer, const float* x, int 
         a.relu = relu;
         a.ev_start = (hipEvent_t)start_event;
         a.ev_stop = (hipEvent_t)stop_event;
-        forward_rows(*layer->layer, a, m, s ? (hipStream_t)s : stream(), staging_scratch);
+        const hipStream_t st = s ? (hipStream_t)s : stream();
+        forward_rows(*layer->layer, a, m, st, staging_scratch, 0);
         return 0;
     });
 }
