@@ -1449,6 +1449,11 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_rows_kernel(
     }
 }
 
+// Query rows from which the matrix cores take Trit's attention
+// (attention_rows.hip: tiles of 16 rows) from the vector kernel's 4 rows a
+// block.
+constexpr int ROWS_MFMA_MIN = 9;
+
 // Shared memory of attention_rows_kernel for R rows over tk keys.
 size_t rows_lds(int R, int tk) {
     return (size_t)(R * MAX_HD + R * ((tk + 3) & ~3) + R * (ATT_THREADS / 64) + R) * 4;
@@ -1493,13 +1498,18 @@ __global__ void rows_to_cache_kernel(const float* __restrict__ k, const float* _
 }  // namespace
 
 // Trit's attention over device rows (q rows of stride qs; k, v rows of
-// stride kvs): the rows go into head-major caches kc, vc (kv_heads x tk x
-// hd floats each) and the exact kernel runs per (head, query row). `st`
-// holds pos = tk - tq and done = 0.
+// stride kvs): on the matrix cores from the rows as they lie; for shapes
+// those do not take, the rows go into head-major caches kc, vc (kv_heads x
+// tk x hd floats each) for the vector kernels. `st` holds pos = tk - tq and
+// done = 0.
 void exact_attention(const float* q, int qs, const float* k, const float* v, int kvs, int tq, int tk, int heads,
                      int kv_heads, int hd, int causal, float* out, float* kc, float* vc, State* st, hipStream_t s) {
     if ((size_t)(MAX_HD + tk + ATT_THREADS) * 4 > 64 * 1024)
         fail("attention: more keys than the exact kernel's shared memory holds (16000)");
+    if (tq >= ROWS_MFMA_MIN && ((uintptr_t)k | (uintptr_t)v) % 16 == 0 &&
+        attention_rows_mfma(RowsArgs{q, qs, heads, kv_heads, k, v, (size_t)hd, (size_t)kvs, tq, tq, causal, out, st},
+                            hd, false, tk, s))
+        return;
     const int grid = (int)std::min<size_t>(4096, ((size_t)tk * kv_heads * hd + 255) / 256);
     hipLaunchKernelGGL(rows_to_cache_kernel<float>, dim3(grid), dim3(256), 0, s, k, v, kvs, tk, kv_heads, hd, kc, vc);
     if (!launch_attention_rows<float>(q, qs, heads, kv_heads, hd, kc, vc, tk, tq, tk, out, st, causal, s)) {
@@ -1508,6 +1518,20 @@ void exact_attention(const float* q, int qs, const float* k, const float* v, int
                            hd, kc, vc, tk, tq, out, 1, st, causal);
     }
     TRIT_HIP(hipGetLastError());
+}
+
+void exact_attention_windows(const float* q, int qs, const float* k, const float* v, int kvs, int rows, int window,
+                             int heads, int hd, float* out, float* kc, float* vc, State* st, hipStream_t s) {
+    const int most = std::min(window, rows);
+    if (most >= ROWS_MFMA_MIN && ((uintptr_t)k | (uintptr_t)v) % 16 == 0 &&
+        attention_rows_mfma(RowsArgs{q, qs, heads, heads, k, v, (size_t)hd, (size_t)kvs, rows, most, 0, out, st}, hd,
+                            false, most, s))
+        return;
+    for (int w0 = 0; w0 < rows; w0 += window) {
+        const int n = std::min(window, rows - w0);
+        exact_attention(q + (size_t)w0 * qs, qs, k + (size_t)w0 * kvs, v + (size_t)w0 * kvs, kvs, n, n, heads, heads,
+                        hd, 0, out + (size_t)w0 * heads * hd, kc, vc, st, s);
+    }
 }
 
 // ---- host side ------------------------------------------------------------
@@ -1740,15 +1764,23 @@ void forward(SessionImpl& S, int rows, hipStream_t s) {
             // The host sizes shared memory for the largest key count this forward can see.
             const size_t lds = (size_t)(MAX_HD + S.max_pos + ATT_THREADS) * 4;
             const size_t lo = (size_t)l * c.kv_heads * S.max_pos * hd;
-            const bool multi =
-                rows > 1 && (S.kv32 ? launch_attention_rows<float>(S.qkv.as<float>(), stride, c.heads, c.kv_heads, hd,
+            // (Many rows are never inside the captured step: the host knows their position.)
+            const void* kl = S.kv32 ? (const void*)(S.kcache.as<float>() + lo) : S.kcache.as<_Float16>() + lo;
+            const void* vl = S.kv32 ? (const void*)(S.vcache.as<float>() + lo) : S.vcache.as<_Float16>() + lo;
+            const bool mfma = rows >= ROWS_MFMA_MIN &&
+                              attention_rows_mfma(RowsArgs{S.qkv.as<float>(), stride, c.heads, c.kv_heads, kl, vl,
+                                                           (size_t)S.max_pos * hd, (size_t)hd, rows, rows, 1,
+                                                           S.att.as<float>(), st},
+                                                  hd, !S.kv32, S.host_pos + rows, s);
+            const bool multi = mfma ||
+                (rows > 1 && (S.kv32 ? launch_attention_rows<float>(S.qkv.as<float>(), stride, c.heads, c.kv_heads, hd,
                                                                   S.kcache.as<float>() + lo, S.vcache.as<float>() + lo,
                                                                   S.max_pos, rows, S.max_pos, S.att.as<float>(), st,
                                                                   1, s)
                                     : launch_attention_rows<_Float16>(
                                           S.qkv.as<float>(), stride, c.heads, c.kv_heads, hd,
                                           S.kcache.as<_Float16>() + lo, S.vcache.as<_Float16>() + lo, S.max_pos,
-                                          rows, S.max_pos, S.att.as<float>(), st, 1, s));
+                                          rows, S.max_pos, S.att.as<float>(), st, 1, s)));
             if (multi) {
                 // R query rows a block.
             } else if (rows == 1 && hd <= MAX_HD && ATT_THREADS % hd == 0 && attention_one_lds(S.max_pos) <= 64 * 1024) {

@@ -101,11 +101,36 @@ void flash_prefill(SessionImpl& S, int layer, int rows, int pos0, hipStream_t s)
 void flash_attention(const float* q, int qs, const _Float16* kc, const _Float16* vc, int max_pos, int heads,
                      int kv_heads, int rows, int pos0, int tk, int causal, float* out, hipStream_t s);
 
+// Trit's attention (its serial orders, every sum exact in its order) of many
+// query rows on the f32 matrix cores (attention_rows.hip): rows of q (stride
+// q_stride) at positions st->pos .., keys and values f32 or f16 of row
+// stride pos_stride, key/value head g at g * head_stride. window: the rows
+// (and the keys, pos 0) fall into windows of that many, each attending to
+// itself; rows for all rows over st->pos + rows keys. tiles, window_tiles
+// are the launch's own.
+struct RowsArgs {
+    const float* q;
+    int q_stride, heads, kvh;
+    const void *k, *v;
+    size_t head_stride, pos_stride;
+    int rows, window, causal;
+    float* out;
+    const State* st;
+    int tiles, window_tiles;
+};
+// False when it does not take the shape: head_dim 64 or 128, at most 3200
+// keys a row (max_tk), strides a multiple of 4 (k and v 16-byte aligned).
+bool attention_rows_mfma(RowsArgs a, int hd, bool f16, int max_tk, hipStream_t s);
+
 // Trit's attention (exact kernel) over device rows: q rows of stride qs,
 // k and v rows of stride kvs; kc / vc scratch of kv_heads x tk x hd floats;
 // st a device State with pos = tk - tq, done = 0 (decoder.hip).
 void exact_attention(const float* q, int qs, const float* k, const float* v, int kvs, int tq, int tk, int heads,
                      int kv_heads, int hd, int causal, float* out, float* kc, float* vc, State* st, hipStream_t s);
+// The same within windows of `window` rows, each attending to itself only
+// (every head its own keys and values, no mask).
+void exact_attention_windows(const float* q, int qs, const float* k, const float* v, int kvs, int rows, int window,
+                             int heads, int hd, float* out, float* kc, float* vc, State* st, hipStream_t s);
 
 // The persistent decode step (decode_step.hip).
 // Whether the session's model and mode run on it.

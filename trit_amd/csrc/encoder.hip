@@ -534,12 +534,9 @@ int trit_hip_asr_encoder_encode(const TritHipAsrEncoder* encoder, const float* m
             hipLaunchKernelGGL(layer_norm_kernel, dim3(t), dim3(64), 0, s, x.as<float>(), d, e.norm(l, 0),
                                e.norm(l, 1), NORM_EPS, xn.as<float>());
             encoder_product(*e.layers[4 * l], xn.as<float>(), t, qkv.as<float>(), nullptr, scratch, s);
-            for (int w0 = 0; w0 < t; w0 += window) {
-                const int n = std::min(window, t - w0);
-                const float* q = qkv.as<float>() + (size_t)w0 * 3 * d;
-                exact_attention(q, 3 * d, q + d, q + 2 * d, 3 * d, n, n, c.heads, c.heads, hd, 0,
-                                att.as<float>() + (size_t)w0 * d, kc.as<float>(), vc.as<float>(), st.as<State>(), s);
-            }
+            exact_attention_windows(qkv.as<float>(), 3 * d, qkv.as<float>() + d, qkv.as<float>() + 2 * d, 3 * d, t,
+                                    window, c.heads, hd, att.as<float>(), kc.as<float>(), vc.as<float>(),
+                                    st.as<State>(), s);
             encoder_product(*e.layers[4 * l + 1], att.as<float>(), t, x.as<float>(), x.as<float>(), scratch, s);
             hipLaunchKernelGGL(layer_norm_kernel, dim3(t), dim3(64), 0, s, x.as<float>(), d, e.norm(l, 2),
                                e.norm(l, 3), NORM_EPS, xn.as<float>());
