@@ -26,10 +26,12 @@
 //
 // Bound: the f32 matrix rate (139 TFLOP/s in a register-only loop) and, one
 // block a CU, the serial sum of phase 3 (about 10 cycles a key); 2-3 blocks a
-// CU overlap each other's phases. Whisper large-v3's layer (1500 rows, 20
-// heads of 64, 11.5 GFLOP): 278 us against 782 us for the vector kernel's 4
-// rows a block; a causal prompt of 1564 rows (16 heads of 128, 10 GFLOP of
-// visible keys): 215 us against 494 us; 256 rows of it 20.7 us against 23.6.
+// CU overlap each other's phases. Vector instructions share the SIMDs with the
+// MFMAs, so addresses are 32-bit offsets and only tiles at an edge are masked
+// (with 64-bit row addresses and a mask a value, 278 us and 210 us below).
+// Whisper large-v3's layer (1500 rows, 20 heads of 64, 11.5 GFLOP): 232 us
+// against 782 us for the vector kernel's 4 rows a block; a causal prompt of 1564
+// rows (16 heads of 128, 10 GFLOP of visible keys): 186 us against 494 us.
 #include <algorithm>
 #include <cmath>
 
@@ -73,7 +75,7 @@ struct alignas(sizeof(KV) * VE) Values {
 };
 
 template <typename KV, int HD, int NT, int W>
-__global__ __launch_bounds__(64 * W, 2) void attention_rows_mfma_kernel(RowsArgs a) {
+__global__ __launch_bounds__(64 * W, W == 4 && (HD == 64 || sizeof(KV) == 2) ? 3 : 2) void attention_rows_mfma_kernel(RowsArgs a) {
     constexpr int VE = HD / TILE > W ? HD / TILE / W : 1;  // 16-dim output tiles a wave
     constexpr int PVW = HD / TILE / VE;                    // waves with output tiles
     constexpr int CT = 4 * W;                              // tiles a chunk
@@ -105,8 +107,11 @@ __global__ __launch_bounds__(64 * W, 2) void attention_rows_mfma_kernel(RowsArgs
     const int t = threadIdx.x;
     const int lane = t % WAVE, w = __builtin_amdgcn_readfirstlane(t / WAVE);
     const int lr = lane % 16, q = lane / 16;
-    const KV* K = (const KV*)a.k + (size_t)g * a.head_stride + (size_t)first * a.pos_stride;
-    const KV* V = (const KV*)a.v + (size_t)g * a.head_stride + (size_t)first * a.pos_stride;
+    // Keys and values at 32-bit byte offsets from the head's first (the host
+    // checks they fit).
+    const char* K = (const char*)((const KV*)a.k + (size_t)g * a.head_stride + (size_t)first * a.pos_stride);
+    const char* V = (const char*)((const KV*)a.v + (size_t)g * a.head_stride + (size_t)first * a.pos_stride);
+    const uint32_t pitch = (uint32_t)(a.pos_stride * sizeof(KV));
 
     // 1. Scores. Operand register i of a lane: dim 4 i + q of query row lr
     // (rows past nr repeat the last one; nothing of them is stored).
@@ -117,14 +122,17 @@ __global__ __launch_bounds__(64 * W, 2) void attention_rows_mfma_kernel(RowsArgs
 #pragma unroll
         for (int i = 0; i < HD / 4; ++i) qf[i] = qr[4 * i] * scale;
     }
-    const int visible = a.causal ? pos + row0 + lr + 1 : tk;
+    const int visible = a.causal ? pos + row0 + lr + 1 : tk;       // of row lr
+    const int all_visible = a.causal ? pos + row0 + 1 : tk;        // of every row
     float s[NT][4];  // s[j][r]: key 16 (w + W j) + 4 q + r of row lr
     float best = -INFINITY;
     Four<KV> next[HD / 16];
+    const uint32_t key_off = (uint32_t)(TILE * w + lr) * pitch, last_off = (uint32_t)(kmax - 1) * pitch;
     auto fetch = [&](int j) {
-        const KV* kr = K + (size_t)min(TILE * (w + W * j) + lr, kmax - 1) * a.pos_stride + 4 * q;
+        // (Past the last key: that key again; its scores are masked.)
+        const uint32_t off = min(key_off + (uint32_t)(TILE * W * j) * pitch, last_off) + 4 * q * (uint32_t)sizeof(KV);
 #pragma unroll
-        for (int i = 0; i < HD / 16; ++i) load4(kr + 16 * i, next[i]);
+        for (int i = 0; i < HD / 16; ++i) load4((const KV*)(K + off) + 16 * i, next[i]);
     };
     fetch(0);
 #pragma unroll
@@ -144,10 +152,14 @@ __global__ __launch_bounds__(64 * W, 2) void attention_rows_mfma_kernel(RowsArgs
 #pragma unroll
                 for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(f[u], qf[4 * i + u], acc, 0, 0, 0);
             }
+            if (key0 + TILE > all_visible) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[r] = key0 + 4 * q + r < visible ? acc[r] : -INFINITY;
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                s[j][r] = key0 + 4 * q + r < visible ? acc[r] : -INFINITY;
-                best = __builtin_fmaxf(best, s[j][r]);
+                s[j][r] = acc[r];
+                best = __builtin_fmaxf(best, acc[r]);
             }
         } else {
 #pragma unroll
@@ -155,7 +167,7 @@ __global__ __launch_bounds__(64 * W, 2) void attention_rows_mfma_kernel(RowsArgs
         }
     }
 
-    // 2. Row lr's maximum, the exponentials (0 past kend).
+    // 2. Row lr's maximum.
     best = __builtin_fmaxf(best, __shfl_xor(best, 16));
     best = __builtin_fmaxf(best, __shfl_xor(best, 32));
     if (q == 0) red[w][lr] = best;
@@ -164,20 +176,23 @@ __global__ __launch_bounds__(64 * W, 2) void attention_rows_mfma_kernel(RowsArgs
 #pragma unroll
     for (int i = 1; i < W; ++i) mx = __builtin_fmaxf(mx, red[i][lr]);
 
-    // 3. The sums over the keys before kmax, in order. Chunk c holds the
-    // tiles W (4 c) .. W (4 c + 4) - 1; in a tile, lane (row, quarter) holds
-    // the keys 4 q .. 4 q + 3.
+    // 3. The exponentials, and the sums over the keys before kmax, in order.
+    // Chunk c holds the tiles W (4 c) .. W (4 c + 4) - 1; in a tile, lane (row,
+    // quarter) holds the keys 4 q .. 4 q + 3.
     float sum = 0.0f;
     auto add_chunk = [&](int c) {
-        const int n = min(CT, ntiles - CT * c);
-        const float4* b = buf[c & 1];
+        const int keys = min(TILE * CT, kmax - TILE * CT * c);  // may be none, when kmax < kend
+        const float4* b = buf[c & 1] + lr;
         float4 cur[4], nxt[4];
+        if (keys >= TILE) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) cur[i] = b[16 * i + lr];
-        for (int i = 0; i < n; ++i) {
-            const int o = min(i + 1, n - 1) * WAVE;
+            for (int u = 0; u < 4; ++u) cur[u] = b[16 * u];
+        }
+        int i = 0;
+        for (; TILE * (i + 1) <= keys; ++i) {
+            const int o = (i + 1) % CT * WAVE;  // (past the keys: any tile, not added)
 #pragma unroll
-            for (int u = 0; u < 4; ++u) nxt[u] = b[o + 16 * u + lr];
+            for (int u = 0; u < 4; ++u) nxt[u] = b[o + 16 * u];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 sum = sum + cur[u].x;
@@ -188,6 +203,7 @@ __global__ __launch_bounds__(64 * W, 2) void attention_rows_mfma_kernel(RowsArgs
 #pragma unroll
             for (int u = 0; u < 4; ++u) cur[u] = nxt[u];
         }
+        for (int k = TILE * i; k < keys; ++k) sum = sum + ((const float*)(b + i * WAVE + k / 4 % 4 * 16))[k % 4];
     };
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
@@ -196,14 +212,9 @@ __global__ __launch_bounds__(64 * W, 2) void attention_rows_mfma_kernel(RowsArgs
             for (int u = 0; u < 4; ++u) {
                 const int j = 4 * c + u;
                 if (j < NT) {
-                    const int key = TILE * (w + W * j) + 4 * q;
-                    float e[4];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        s[j][r] = key + r < kend ? exp_trit(s[j][r] - mx) : 0.0f;
-                        e[r] = key + r < kmax ? s[j][r] : 0.0f;
-                    }
-                    buf[c & 1][(u * W + w) * WAVE + lane] = make_float4(e[0], e[1], e[2], e[3]);
+                    for (int r = 0; r < 4; ++r) s[j][r] = exp_trit(s[j][r] - mx);
+                    buf[c & 1][(u * W + w) * WAVE + lane] = make_float4(s[j][0], s[j][1], s[j][2], s[j][3]);
                 }
             }
             __syncthreads();  // the chunk is written; the one before it is added up
@@ -214,20 +225,36 @@ __global__ __launch_bounds__(64 * W, 2) void attention_rows_mfma_kernel(RowsArgs
     __syncthreads();
     const float inv = inv_of[lr];
 
-    // 4. Outputs: register i of the operand is key 4 i + q of the tile; the
-    // pad of the last tile is 0 times -0, which leaves every chain as it is.
+    // 4. Outputs: register i of the operand is key 4 i + q of the tile. The
+    // values past kend are -0: with any finite weight that leaves every chain
+    // as it is.
     f32x4 out[VE];
 #pragma unroll
     for (int u = 0; u < VE; ++u) out[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const bool chains = w < PVW;
-    const int e0 = VE * (TILE * (chains ? w : 0) + lr);  // the lane's first dim
+    const uint32_t dim_off = (uint32_t)(VE * (TILE * (chains ? w : 0) + lr)) * (uint32_t)sizeof(KV);
+    const uint32_t lane_off = (uint32_t)q * pitch + dim_off;
+    // Groups of four tiles, all but the last of whole tiles; nv: a group's values.
+    const int whole = kend / (4 * TILE);
     Values<KV, VE> nv[16];
-    auto fetch_values = [&](int tile0) {
+    auto fetch_value = [&](int group, int i) {
+        const uint32_t at = (uint32_t)(4 * (16 * group + i)) * pitch;
+        nv[i] = *(const Values<KV, VE>*)(V + at + lane_off);
+    };
+    auto fetch_last = [&](int group) {
+        const uint32_t end = (uint32_t)(kend - 1) * pitch;
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-            nv[i] = *(const Values<KV, VE>*)(V + (size_t)min(TILE * tile0 + 4 * i + q, kend - 1) * a.pos_stride + e0);
+            nv[i] = *(const Values<KV, VE>*)(V + min((uint32_t)(4 * (16 * group + i) + q) * pitch, end) + dim_off);
     };
-    if (chains) fetch_values(0);
+    if (chains) {
+        if (whole > 0) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) fetch_value(0, i);
+        } else {
+            fetch_last(0);
+        }
+    }
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
         if (CT * c < ntiles) {
@@ -247,22 +274,39 @@ __global__ __launch_bounds__(64 * W, 2) void attention_rows_mfma_kernel(RowsArgs
                 const int n = min(CT, ntiles - CT * c);
 #pragma unroll 1
                 for (int i = 0; i < n; i += 4) {
-                    Values<KV, VE> cv[16];
+                    const int group = CT / 4 * c + i / 4;
+                    const float4* b = buf[c & 1] + i * WAVE + lane;
+                    if (group < whole) {
+                        const bool more = group + 1 < whole;
 #pragma unroll
-                    for (int u = 0; u < 16; ++u) cv[u] = nv[u];
-                    if (CT * c + i + 4 < ntiles) fetch_values(CT * c + i + 4);
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        if (i + u < n) {
-                            const float4 p4 = buf[c & 1][(i + u) * WAVE + lane];
+                        for (int u = 0; u < 4; ++u) {
+                            const float4 p4 = b[u * WAVE];
                             const float p[4] = {p4.x, p4.y, p4.z, p4.w};
-                            const int key = TILE * (CT * c + i + u) + q;
+#pragma unroll
+                            for (int x = 0; x < 4; ++x)
+#pragma unroll
+                                for (int v = 0; v < VE; ++v)
+                                    out[v] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)nv[4 * u + x].e[v], p[x], out[v],
+                                                                                  0, 0, 0);
+                            if (more) {
+#pragma unroll
+                                for (int x = 0; x < 4; ++x) fetch_value(group + 1, 4 * u + x);
+                            }
+                        }
+                        if (!more && 4 * group + 4 < ntiles) fetch_last(group + 1);
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            if (i + u >= n) break;
+                            const float4 p4 = b[u * WAVE];
+                            const float p[4] = {p4.x, p4.y, p4.z, p4.w};
 #pragma unroll
                             for (int x = 0; x < 4; ++x)
 #pragma unroll
                                 for (int v = 0; v < VE; ++v) {
-                                    const float val = key + 4 * x < kend ? (float)cv[4 * u + x].e[v] : -0.0f;
-                                    out[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(val, p[x], out[v], 0, 0, 0);
+                                    const bool in = 4 * (16 * group + 4 * u + x) + q < kend;
+                                    out[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? (float)nv[4 * u + x].e[v] : -0.0f,
+                                                                                  p[x], out[v], 0, 0, 0);
                                 }
                         }
                     }
@@ -282,7 +326,7 @@ __global__ __launch_bounds__(64 * W, 2) void attention_rows_mfma_kernel(RowsArgs
             if (kend < tk && !(__builtin_fabsf(acc) >= 0x1p-80f)) {
                 const float pm = exp_trit(-INFINITY) * inv;
                 for (int key = kend; key < tk; ++key)
-                    acc = __builtin_fmaf(pm, (float)V[(size_t)key * a.pos_stride + e], acc);
+                    acc = __builtin_fmaf(pm, (float)((const KV*)(V + (uint32_t)key * pitch))[e], acc);
             }
             o[e] = acc;
         }
@@ -314,6 +358,8 @@ bool attention_rows_mfma(RowsArgs a, int hd, bool f16, int max_tk, hipStream_t s
     a.window_tiles = (std::min(a.window, a.rows) + TILE - 1) / TILE;
     a.tiles = a.rows / a.window * a.window_tiles + (a.rows % a.window + TILE - 1) / TILE;
     if ((int64_t)a.tiles * a.heads > (1 << 30)) return false;
+    // 32-bit byte offsets of a tile past the last key.
+    if ((max_tk + 8 * TILE * 32) * (int64_t)a.pos_stride * (f16 ? 2 : 4) >= (int64_t)1 << 31) return false;
     if (f16) return hd == 64 ? launch_hd<_Float16, 64>(a, max_tk, s) : launch_hd<_Float16, 128>(a, max_tk, s);
     return hd == 64 ? launch_hd<float, 64>(a, max_tk, s) : launch_hd<float, 128>(a, max_tk, s);
 }
