@@ -306,6 +306,79 @@ __global__ void qk_rope_kernel(float* __restrict__ qkv, int stride, int heads, i
     }
 }
 
+// The same for many rows, RH heads a block: their values in LDS, one thread a
+// head running Trit's serial sum (a block a head left 127 of 128 threads idle
+// through it and its barriers: 1564 rows of 32 heads of 128 took 32.5 us, here 18.4), then
+// all threads the rotary pairs.
+constexpr int RH = 32;
+
+template <typename KV>
+__global__ __launch_bounds__(256) void qk_rope_rows_kernel(float* __restrict__ qkv, int stride, int rows, int heads,
+                                                           int kvh, int hd, int qk_norm,
+                                                           const float* __restrict__ q_norm,
+                                                           const float* __restrict__ k_norm, float eps,
+                                                           const float* __restrict__ rope_sin,
+                                                           const float* __restrict__ rope_cos,
+                                                           KV* __restrict__ kcache, KV* __restrict__ vcache,
+                                                           int max_pos, const State* st) {
+    if (st->done) return;
+    extern __shared__ __align__(16) float vals[];  // [RH][hd + 4], then RH factors
+    const int pitch = hd + 4, half = hd / 2;
+    float* inv_of = vals + RH * pitch;
+    const int per_row = heads + 2 * kvh, item0 = blockIdx.x * RH;
+    const int items = min(RH, rows * per_row - item0);
+    for (int i = threadIdx.x; i < items * (hd / 4); i += 256) {
+        const int it = i / (hd / 4), e = (i - it * (hd / 4)) * 4;
+        const int row = (item0 + it) / per_row, head = (item0 + it) - row * per_row;
+        const float* src = qkv + (size_t)row * stride + (size_t)head * hd + e;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) vals[it * pitch + e + u] = src[u];
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < items) {
+        const float* v = vals + threadIdx.x * pitch;
+        float sum = 0.0f;
+        if (qk_norm)
+            for (int e = 0; e < hd; e += 8) {
+                const float4 a = *(const float4*)(v + e), b = *(const float4*)(v + e + 4);
+                const float q[8] = {a.x * a.x, a.y * a.y, a.z * a.z, a.w * a.w, b.x * b.x, b.y * b.y, b.z * b.z, b.w * b.w};
+#pragma unroll
+                for (int u = 0; u < 8; ++u) sum = sum + q[u];
+            }
+        inv_of[threadIdx.x] = 1.0f / __builtin_sqrtf(sum / (float)hd + eps);
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < items * half; p += 256) {
+        const int it = p / half, i = p - it * half;
+        const int row = (item0 + it) / per_row, head = (item0 + it) - row * per_row;
+        const bool is_q = head < heads, is_k = !is_q && head < heads + kvh;
+        const int pos = st->pos + row;
+        float a = vals[it * pitch + i], b = vals[it * pitch + i + half];
+        if (is_q || is_k) {
+            if (qk_norm) {
+                const float* w = is_q ? q_norm : k_norm;
+                const float f = inv_of[it];
+                a = a * (f * w[i]);
+                b = b * (f * w[i + half]);
+            }
+            const float s = rope_sin[(size_t)pos * half + i], c = rope_cos[(size_t)pos * half + i];
+            const float ac = a * c, bs = b * s, bc = b * c, as = a * s;
+            a = ac - bs;
+            b = bc + as;
+        }
+        if (is_q) {
+            float* dst = qkv + (size_t)row * stride + (size_t)head * hd;
+            dst[i] = a;
+            dst[i + half] = b;
+        } else {
+            KV* cache = is_k ? kcache : vcache;
+            KV* dst = cache + ((size_t)(head - heads - (is_k ? 0 : kvh)) * max_pos + pos) * hd;
+            dst[i] = (KV)a;
+            dst[i + half] = (KV)b;
+        }
+    }
+}
+
 // Fast mode, head_dim 128: the same step with one wave per (row, head),
 // lane i holding dims i and i + 64 (a rotary pair), the norm's sum a DPP
 // tree (fast mode: tree sums) -- four heads a 256-thread block instead of
@@ -1179,8 +1252,7 @@ __device__ __forceinline__ void attention_one(float* sm, const float* __restrict
     float* qh = sm + ONE_VB / 4;
     float* probs = qh + MAX_HD;
     float* red = probs + ((tk + 3) & ~3);
-    const KV* K = kcache + (size_t)g * max_pos * hd;
-    const KV* V = vcache + (size_t)g * max_pos * hd;
+    const int per_key = hd * (int)sizeof(KV) / 16;  // pieces
     constexpr int PIECES = ONE_VB / 16 / ATT_THREADS;
     uint4 vr[PIECES];
     auto load_stage = [&](int s0) {
@@ -1199,7 +1271,7 @@ __device__ __forceinline__ void attention_one(float* sm, const float* __restrict
     float best = -INFINITY;
     for (int j = t; j < tk; j += ATT_THREADS) {
         float acc = 0.0f;
-        const KV* kr = K + (size_t)j * hd;
+        const KV* kr = K + (size_t)j * stride;
         if constexpr (HD > 0) {
             float kv[HD];
 #pragma unroll
@@ -1353,7 +1425,8 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_rows_kernel(
         qh[r * MAX_HD + e] = r < nr ? qkv[(size_t)(row0 + r) * stride + (size_t)h * hd + e] * scale : 0.0f;
     }
     __syncthreads();
-    const int per_key = hd * (int)sizeof(KV) / 16;  // pieces
+    const KV* K = kcache + (size_t)g * max_pos * hd;
+    const KV* V = vcache + (size_t)g * max_pos * hd;
     float best[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) best[r] = -INFINITY;
@@ -1361,7 +1434,7 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_rows_kernel(
         float acc[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-        const KV* kr = K + (size_t)j * stride;
+        const KV* kr = K + (size_t)j * hd;
         for (int e = 0; e < hd; e += 8) {
             float kv[8];
             kv_load8(kr + e, kv);
@@ -1767,35 +1840,33 @@ void forward(SessionImpl& S, int rows, hipStream_t s) {
         // q/k norm, rotary, cache append, attention.
         const bool fused = !S.exact && rows == 1 && q_scale == 1.0f;
         if (!fused) {
-            if (S.exact && !S.kv32) {
-                // Trit's serial q/k norm sums, f16 caches.
-                hipLaunchKernelGGL(qk_rope_kernel<_Float16>, dim3(rows * (c.heads + 2 * c.kv_heads)),
-                                   dim3(hd < 64 ? 64 : hd), 0, s, S.qkv.as<float>(), stride, c.heads, c.kv_heads, hd,
-                                   c.qk_norm, D.q_norm(l), D.k_norm(l), c.eps, S.rope_sin.as<float>(),
-                                   S.rope_cos.as<float>(),
-                                   S.kcache.as<_Float16>() + (size_t)l * c.kv_heads * S.max_pos * hd,
-                                   S.vcache.as<_Float16>() + (size_t)l * c.kv_heads * S.max_pos * hd, S.max_pos, st);
-            } else if (S.kv32) {
-                hipLaunchKernelGGL(qk_rope_kernel<float>, dim3(rows * (c.heads + 2 * c.kv_heads)),
-                                   dim3(hd < 64 ? 64 : hd), 0, s, S.qkv.as<float>(), stride, c.heads, c.kv_heads, hd,
-                                   c.qk_norm, D.q_norm(l), D.k_norm(l), c.eps, S.rope_sin.as<float>(),
-                                   S.rope_cos.as<float>(),
-                                   S.kcache.as<float>() + (size_t)l * c.kv_heads * S.max_pos * hd,
-                                   S.vcache.as<float>() + (size_t)l * c.kv_heads * S.max_pos * hd, S.max_pos, st);
-            } else if (hd == 128 && use_qk_wave()) {
+            // Trit's serial q/k norm sums, but for the fast mode's f16 caches at head_dim 128.
+            const auto rope = [&](auto* kc, auto* vc) {
+                using KV = std::remove_pointer_t<decltype(kc)>;
+                const size_t lo = (size_t)l * c.kv_heads * S.max_pos * hd;
+                const int items = rows * (c.heads + 2 * c.kv_heads);
+                if (rows > 1)
+                    hipLaunchKernelGGL(qk_rope_rows_kernel<KV>, dim3((items + RH - 1) / RH), dim3(256),
+                                       (size_t)(RH * (hd + 4) + RH) * 4, s, S.qkv.as<float>(), stride, rows, c.heads,
+                                       c.kv_heads, hd, c.qk_norm, D.q_norm(l), D.k_norm(l), c.eps,
+                                       S.rope_sin.as<float>(), S.rope_cos.as<float>(), kc + lo, vc + lo, S.max_pos, st);
+                else
+                    hipLaunchKernelGGL(qk_rope_kernel<KV>, dim3(items), dim3(hd < 64 ? 64 : hd), 0, s,
+                                       S.qkv.as<float>(), stride, c.heads, c.kv_heads, hd, c.qk_norm, D.q_norm(l),
+                                       D.k_norm(l), c.eps, S.rope_sin.as<float>(), S.rope_cos.as<float>(), kc + lo,
+                                       vc + lo, S.max_pos, st);
+            };
+            if (!S.exact && !S.kv32 && hd == 128 && use_qk_wave()) {
                 const int items = rows * (c.heads + 2 * c.kv_heads);
                 hipLaunchKernelGGL(qk_rope_wave_kernel<_Float16>, dim3((items + 3) / 4), dim3(256), 0, s,
                                    S.qkv.as<float>(), stride, rows, c.heads, c.kv_heads, c.qk_norm, D.q_norm(l),
                                    D.k_norm(l), c.eps, S.rope_sin.as<float>(), S.rope_cos.as<float>(),
                                    S.kcache.as<_Float16>() + (size_t)l * c.kv_heads * S.max_pos * hd,
                                    S.vcache.as<_Float16>() + (size_t)l * c.kv_heads * S.max_pos * hd, S.max_pos, st);
+            } else if (S.kv32) {
+                rope(S.kcache.as<float>(), S.vcache.as<float>());
             } else {
-                hipLaunchKernelGGL(qk_rope_kernel<_Float16>, dim3(rows * (c.heads + 2 * c.kv_heads)),
-                                   dim3(hd < 64 ? 64 : hd), 0, s, S.qkv.as<float>(), stride, c.heads, c.kv_heads, hd,
-                                   c.qk_norm, D.q_norm(l), D.k_norm(l), c.eps, S.rope_sin.as<float>(),
-                                   S.rope_cos.as<float>(),
-                                   S.kcache.as<_Float16>() + (size_t)l * c.kv_heads * S.max_pos * hd,
-                                   S.vcache.as<_Float16>() + (size_t)l * c.kv_heads * S.max_pos * hd, S.max_pos, st);
+                rope(S.kcache.as<_Float16>(), S.vcache.as<_Float16>());
             }
             TRIT_HIP(hipGetLastError());
             if (q_scale != 1.0f)
