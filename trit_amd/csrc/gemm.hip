@@ -1,6 +1,6 @@
 // Integer products of many rows (prompt prefill) on the matrix cores:
-// Q8_0 (and Q4_K requantized to it) with 32-value groups, Trit int8 with
-// 128-value groups.
+// Q8_0 (and Q4_K requantized to it) with 32-value groups, Trit int8 and
+// ternary with 128-value groups.
 //
 // The values are Trit's, bit for bit, as in the small-batch kernels
 // (src/cpu/int8.rs:525-584, src/cpu/v2/product.rs:389-423):
@@ -30,11 +30,37 @@
 #include "device.h"
 #include "internal.h"
 
+#include <type_traits>
+
 namespace trit {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
+
+__device__ __forceinline__ v16f lower(const v32f& v) {
+    return __builtin_shufflevector(v, v, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+}
+__device__ __forceinline__ v16f upper(const v32f& v) {
+    return __builtin_shufflevector(v, v, 16, 17, 18, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28, 29, 30, 31);
+}
+
+// Dots from the matrix cores as f32: accumulated on 0x4b400000, the bits of
+// 1.5 * 2^23, a dot d is the bits of 1.5 * 2^23 + d exactly (|d| <= 128 * 128 *
+// 127 < 2^22), so one subtraction gives f32(d) -- at nearly twice the rate of
+// the conversion (16 of them 51 cycles a wave against 85, four waves a SIMD).
+__device__ __forceinline__ v16i dot_base() {
+    v16i m;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) m[r] = 0x4b400000;
+    // Sixteen registers, not a constant moved into every accumulator.
+    asm("" : "+v"(m));
+    return m;
+}
+__device__ __forceinline__ float dot_of(int bits) { return __builtin_bit_cast(float, bits) - 12582912.0f; }
 
 constexpr int GEMM_THREADS = 256;
 constexpr int BM = 64;  // rows of x per block: two waves of 32
@@ -633,7 +659,122 @@ __global__ __launch_bounds__(GEMM_THREADS, TW == 2 ? 3 : 4) void gemm_dma_kernel
     }
 }
 
-int group_of(const Layer& L) { return L.kind == INT8 ? 128 : 32; }
+// Ternary products of many rows: 2-bit codes, f32 scales a 128-group, the
+// same contract (dot of the codes minus one and the activation codes). A wave
+// owns 32 x rows by TN 32-row weight tiles, four waves a block (2 x 2); no LDS
+// and no barriers, every operand straight from global memory, three groups in
+// flight. The order of K inside a group is free (an integer dot): MFMA step s
+// of a group takes the codes 64 h + 16 s .. + 15 for the half h of the lanes,
+// so a lane's 16 bytes of 2-bit codes are its four steps' operands, each dword
+// unpacked by shifts, a mask and a byte permute that looks up code - 1. The
+// scale products ws * xs come from the matrix cores as well, the outer product
+// of the two scale vectors in the dots' register layout (one product rounded
+// once, as the vector multiply rounds it), which leaves a conversion and a
+// multiply-add an output to the vector ALUs.
+constexpr int TERN_DEPTH = 3;
+
+template <int TN>
+__global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_ternary_kernel(const int8_t* __restrict__ xq,
+                                                                       const float* __restrict__ xs, int m, int mpad,
+                                                                       const uint8_t* __restrict__ codes,
+                                                                       const float* __restrict__ scales,
+                                                                       const float* __restrict__ bias, int n, int k,
+                                                                       int nb, int mb, GemvArgs a) {
+    if (a.skip && *a.skip) return;
+    const int groups = k / 128;
+    const int blk = blockIdx.x;
+    int bn, bm;
+    if (nb % 8 == 0) {
+        const int q = blk / 8;
+        bn = blk % 8 + 8 * (q / mb);
+        bm = q % mb;
+    } else {
+        bn = blk % nb;
+        bm = blk / nb;
+    }
+    const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int lr = lane % 32, h = lane / 32;
+    const int m0 = bm * BM + 32 * (w % 2), n0 = (bn * 2 + w / 2) * 32 * TN;
+    if (m0 >= m || n0 >= n) return;
+    const int8_t* xp = xq + (size_t)min(m0 + lr, m - 1) * k + 64 * h;
+    const float* xsp = xs + m0 + lr;  // mpad covers the tile's rows
+    const uint8_t* wp[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) wp[j] = codes + (size_t)min(n0 + 32 * j + lr, n - 1) * (k / 4) + 16 * h;
+    // The lane's weight scales: of row lr of tile h (TN = 2) or of the tile.
+    const float* wsp = scales + (size_t)min(n0 + 32 * (TN == 2 ? h : 0) + lr, n - 1) * groups;
+    v4i av[TERN_DEPTH][4];
+    uint4 bv[TERN_DEPTH][TN];
+    float xv[TERN_DEPTH], wv[TERN_DEPTH];
+    auto fetch = [&](int g, int d) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) av[d][s] = *(const v4i*)(xp + (size_t)g * 128 + 16 * s);
+        xv[d] = xsp[(size_t)g * mpad];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) bv[d][j] = *(const uint4*)(wp[j] + (size_t)g * 32);
+        wv[d] = wsp[g];
+    };
+    const v16i magic = dot_base();
+    float t[TN][16];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) t[j][r] = 0.0f;
+#pragma unroll
+    for (int d = 0; d < TERN_DEPTH; ++d)
+        if (d < groups) fetch(d, d);
+    for (int g0 = 0; g0 < groups; g0 += TERN_DEPTH) {
+#pragma unroll
+        for (int d = 0; d < TERN_DEPTH; ++d) {
+            const int g = g0 + d;
+            if (g >= groups) break;
+            v16i dot[TN];
+            v16f sc[TN];
+            if constexpr (TN == 2) {
+                const v32f both = __builtin_amdgcn_mfma_f32_32x32x1f32(xv[d], wv[d], v32f{}, 0, 0, 0);
+                sc[0] = lower(both);
+                sc[1] = upper(both);
+            } else {
+                sc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(h ? 0.0f : xv[d], h ? 0.0f : wv[d], v16f{}, 0, 0, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const uint32_t words[4] = {bv[d][j].x, bv[d][j].y, bv[d][j].z, bv[d][j].w};
+                dot[j] = magic;
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    v4i b;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        b[i] = (int)__builtin_amdgcn_perm(0u, 0x020100FFu, (words[s] >> (2 * i)) & 0x03030303u);
+                    dot[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[d][s], b, dot[j], 0, 0, 0);
+                }
+            }
+            if (g + TERN_DEPTH < groups) fetch(g + TERN_DEPTH, d);
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) t[j][r] = __builtin_fmaf(dot_of(dot[j][r]), sc[j][r], t[j][r]);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int col = n0 + 32 * j + lr;
+        if (col >= n) continue;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = m0 + 8 * (r / 4) + 4 * h + r % 4;
+            if (row >= m) continue;
+            float v = t[j][r];
+            if (bias) v = v + bias[col];
+            if (a.relu) v = __builtin_fmaxf(v, 0.0f);
+            const size_t at = (size_t)row * n + col;
+            a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v : v;
+        }
+    }
+}
+
+int group_of(const Layer& L) { return L.kind == INT8 || L.kind == TERNARY ? 128 : 32; }
 
 struct Scratch {
     int8_t* xq;
@@ -696,10 +837,27 @@ void launch_gemm(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStream
     TRIT_HIP(hipGetLastError());
 }
 
+// Two weight tiles a wave where that still makes a block for every CU, else
+// one.
+void launch_ternary(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStream_t s) {
+    const int mb = sc.mpad / BM;
+    auto go = [&](auto TN_) {
+        constexpr int TN = decltype(TN_)::value;
+        const int nb = (L.n + 64 * TN - 1) / (64 * TN);
+        launch_timed(a, gemm_ternary_kernel<TN>, dim3(nb * mb), dim3(GEMM_THREADS), 0, s, (const int8_t*)sc.xq,
+                     (const float*)sc.xs, a.m, sc.mpad, L.codes.as<uint8_t>(), L.scales.as<float>(),
+                     L.bias.as<float>(), L.n, L.k, nb, mb, a);
+    };
+    if ((int64_t)((L.n + 127) / 128) * mb >= 256) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 1>{});
+    TRIT_HIP(hipGetLastError());
+}
+
 }  // namespace
 
 bool gemm_supported(const Layer& L, const GemvArgs& a) {
-    if (L.kind != Q8_0 && L.kind != Q4_K && L.kind != INT8) return false;
+    if (L.kind != Q8_0 && L.kind != Q4_K && L.kind != INT8 && L.kind != TERNARY) return false;
+    if (L.kind == TERNARY && a.epilogue == EPI_SILU_PAIR) return false;
     // k a multiple of the group (a partial last chunk of K is zero past k);
     // RMSNorm computed here takes whole 256-value chunks.
     if (L.k % group_of(L) != 0) return false;
@@ -736,6 +894,7 @@ void gemm_int(const Layer& L, const GemvArgs& a, void* scratch, hipStream_t s) {
         hipLaunchKernelGGL((quantize_kernel<128, false>), dim3(qblocks), dim3(256), 0, s, a.x, a.m, sc.mpad, L.k,
                            a.norm_w, inv, sc.xq, sc.xs, a.skip);
     TRIT_HIP(hipGetLastError());
+    if (L.kind == TERNARY) return launch_ternary(L, a, sc, s);
     const bool pair = a.epilogue == EPI_SILU_PAIR;
     if (G == 32) {
         if (pair) return launch_gemm<32, true, 2>(L, a, sc, s);

@@ -347,7 +347,24 @@ size_t staging_spare(hipStream_t s) {
 template <class Scratch>
 void forward_rows(const Layer& L, GemvArgs a, int m, hipStream_t s, Scratch get, size_t spare) {
     a.m = m;
-    if (m >= GEMM_MIN_ROWS && gemm_supported(L, a)) return gemm_int(L, a, get(gemm_scratch_bytes(m, L.k)), s);
+    if (m >= GEMM_MIN_ROWS && L.kind == TERNARY) {
+        // Passes of whole 64-row tiles where 64 MiB or `spare` does not hold all rows.
+        const size_t tile = gemm_scratch_bytes(64, L.k);
+        if (!a.ev_start && !a.ev_stop && gemm_supported(L, a) && tile <= spare) {
+            const size_t tiles = std::max<size_t>(1, std::min(spare, (size_t)64 << 20) / tile), all = (size_t)(m + 63) / 64;
+            const int rows = (int)std::min((size_t)m, 64 * std::min(tiles, all));
+            const float* x = a.x;
+            float* y = a.y;
+            for (int r0 = 0; r0 < m; r0 += rows) {
+                a.x = x + (size_t)r0 * L.k;
+                a.y = y + (size_t)r0 * L.n;
+                a.m = m - r0 < rows ? m - r0 : rows;
+                gemm_int(L, a, get(gemm_scratch_bytes(a.m, L.k)), s);
+            }
+            return;
+        }
+    } else if (m >= GEMM_MIN_ROWS && gemm_supported(L, a))
+        return gemm_int(L, a, get(gemm_scratch_bytes(m, L.k)), s);
     if (m > 8 && !a.ev_start && !a.ev_stop && gemm_float_supported(L, a)) return gemm_float(L, a, s);
     if (m > 8 && !a.ev_start && !a.ev_stop && gemm_float_mfma_supported(L, a) &&
         gemm_float_scratch_bytes(1, L.k) <= spare) {
