@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/trit_hip.h"
 #include "decoder_impl.h"
@@ -47,11 +48,77 @@ __global__ void add_kernel(float* __restrict__ x, const float* __restrict__ y, s
         x[i] = x[i] + y[i];
 }
 
-// Norm::apply (src/layers.rs:50-64,84-121), one 64-lane wave a row: lane j
-// < 32 chains the values j, j + 32, ... of the mean's (then the
-// variance's) sum; lane 0 adds the 32 lane sums in order and then the
-// tail; out = (v - mean) * inv * w + b.
-__global__ __launch_bounds__(64) void layer_norm_kernel(const float* __restrict__ x, int d, const float* __restrict__ w,
+// Norm::apply (src/layers.rs:50-64,84-121): chain j < 32 of the mean's (then
+// the variance's) sum runs over the values j, j + 32, ... in order, the 32
+// chains are added in order from 0, then the serial sum of the tail past the
+// last whole 32; out = (v - mean) * inv * w + b. Half a wave a row, lane j
+// chain j: a row's values (d <= 32 NV) load at once into registers and serve
+// both sums and the output. 1500 rows of 1280: 6.2 us, 22.1 us when a wave a
+// row loaded them from memory three times, step by step of its chains.
+constexpr int LN_ROWS = 4;  // rows a block
+
+template <int NV>
+__global__ __launch_bounds__(32 * LN_ROWS) void layer_norm_kernel(const float* __restrict__ x, int rows, int d,
+                                                                  const float* __restrict__ w,
+                                                                  const float* __restrict__ b, float eps,
+                                                                  float* __restrict__ out) {
+    __shared__ __align__(16) float lanes[LN_ROWS][32];
+    const int j = threadIdx.x % 32, slot = threadIdx.x / 32;
+    const int at = blockIdx.x * LN_ROWS + slot;
+    const bool live = at < rows;
+    const float* row = x + (size_t)(live ? at : 0) * d;
+    const int whole = d / 32;
+    const float n = (float)d;
+    float v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = row[32 * min(i, whole - 1) + j];  // past the chain: its last value
+    float stat[2];
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+        const float mean = pass ? stat[0] : 0.0f;
+        float acc = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            // (A chain from +0 is never -0, so + 0 past its end leaves it.)
+            const float u = pass ? (v[i] - mean) * (v[i] - mean) : v[i];
+            acc += i < whole ? u : 0.0f;
+        }
+        lanes[slot][j] = acc;
+        __syncthreads();
+        float s = 0.0f, t = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 32; i += 4) {
+            const float4 l = *(const float4*)&lanes[slot][i];
+            s += l.x;
+            s += l.y;
+            s += l.z;
+            s += l.w;
+        }
+        for (int i = 32 * whole; i < d; ++i) {
+            const float u = row[i];
+            t += pass ? (u - mean) * (u - mean) : u;
+        }
+        stat[pass] = (s + t) / n;
+        __syncthreads();
+    }
+    if (!live) return;
+    const float mean = stat[0];
+    const float inv = 1.0f / __builtin_sqrtf(stat[1] + eps);
+    float* o = out + (size_t)at * d;
+    // (The last value again past the chain: no branch a value, which would
+    // make each wait for its own weights.)
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int e = 32 * min(i, whole - 1) + j;
+        o[e] = (v[i] - mean) * inv * w[e] + b[e];
+    }
+    const int i = 32 * whole + j;
+    if (i < d) o[i] = (row[i] - mean) * inv * w[i] + b[i];
+}
+
+// The same for rows of fewer than 32 values or more than the registers above take, one
+// 64-lane wave a row, the values read again for each sum.
+__global__ __launch_bounds__(64) void layer_norm_wide_kernel(const float* __restrict__ x, int d, const float* __restrict__ w,
                                                         const float* __restrict__ b, float eps, float* __restrict__ out) {
     __shared__ float lanes[32];
     __shared__ float stat[2];
@@ -86,6 +153,22 @@ __global__ __launch_bounds__(64) void layer_norm_kernel(const float* __restrict_
     const float inv = 1.0f / __builtin_sqrtf(stat[1] + eps);
     float* o = out + (size_t)blockIdx.x * d;
     for (int i = lane; i < d; i += 64) o[i] = (row[i] - mean) * inv * w[i] + b[i];
+}
+
+void layer_norm(const float* x, int rows, int d, const float* w, const float* b, float eps, float* out,
+                hipStream_t s) {
+    const auto go = [&](auto NV_) {
+        constexpr int NV = decltype(NV_)::value;
+        hipLaunchKernelGGL(layer_norm_kernel<NV>, dim3((rows + LN_ROWS - 1) / LN_ROWS), dim3(32 * LN_ROWS), 0, s, x, rows,
+                           d, w, b, eps, out);
+    };
+    if (d < 32 || d >= 32 * 65)
+        hipLaunchKernelGGL(layer_norm_wide_kernel, dim3(rows), dim3(64), 0, s, x, d, w, b, eps, out);
+    else if (d < 32 * 17) go(std::integral_constant<int, 16>{});
+    else if (d < 32 * 25) go(std::integral_constant<int, 24>{});
+    else if (d < 32 * 33) go(std::integral_constant<int, 32>{});
+    else if (d < 32 * 41) go(std::integral_constant<int, 40>{});
+    else go(std::integral_constant<int, 64>{});
 }
 
 // AudioEncoder::chunk's first map (src/models/families/qwen3_asr.rs:
@@ -383,21 +466,18 @@ int trit_hip_encoder_encode(const TritHipEncoder* encoder, const float* mel, flo
             const Layer& Lout = *e.layers[4 * l + 1];
             const Layer& Lfc1 = *e.layers[4 * l + 2];
             const Layer& Lfc2 = *e.layers[4 * l + 3];
-            hipLaunchKernelGGL(layer_norm_kernel, dim3(P), dim3(64), 0, s, x.as<float>(), d, e.norm(l, 0),
-                               e.norm(l, 1), NORM_EPS, xn.as<float>());
+            layer_norm(x.as<float>(), P, d, e.norm(l, 0), e.norm(l, 1), NORM_EPS, xn.as<float>(), s);
             encoder_product(Lqkv, xn.as<float>(), P, qkv.as<float>(), nullptr, scratch, s);
             exact_attention(qkv.as<float>(), 3 * d, qkv.as<float>() + d, qkv.as<float>() + 2 * d, 3 * d, P, P, c.heads,
                             c.heads, hd, 0, att.as<float>(), kc.as<float>(), vc.as<float>(), st.as<State>(), s);
             encoder_product(Lout, att.as<float>(), P, x.as<float>(), x.as<float>(), scratch, s);
-            hipLaunchKernelGGL(layer_norm_kernel, dim3(P), dim3(64), 0, s, x.as<float>(), d, e.norm(l, 2),
-                               e.norm(l, 3), NORM_EPS, xn.as<float>());
+            layer_norm(x.as<float>(), P, d, e.norm(l, 2), e.norm(l, 3), NORM_EPS, xn.as<float>(), s);
             encoder_product(Lfc1, xn.as<float>(), P, hid.as<float>(), nullptr, scratch, s);
             hipLaunchKernelGGL(gelu_kernel, dim3(blocks_for((size_t)P * c.ffn)), dim3(256), 0, s, hid.as<float>(),
                                (size_t)P * c.ffn);
             encoder_product(Lfc2, hid.as<float>(), P, x.as<float>(), x.as<float>(), scratch, s);
         }
-        hipLaunchKernelGGL(layer_norm_kernel, dim3(P), dim3(64), 0, s, x.as<float>(), d, e.norm(c.layers, 0),
-                           e.norm(c.layers, 1), NORM_EPS, xn.as<float>());
+        layer_norm(x.as<float>(), P, d, e.norm(c.layers, 0), e.norm(c.layers, 1), NORM_EPS, xn.as<float>(), s);
         TRIT_HIP(hipGetLastError());
         TRIT_HIP(hipMemcpyAsync(out, xn.ptr, (size_t)P * d * 4, hipMemcpyDeviceToHost, s));
         TRIT_HIP(hipStreamSynchronize(s));
@@ -531,23 +611,20 @@ int trit_hip_asr_encoder_encode(const TritHipAsrEncoder* encoder, const float* m
                            e.positions.as<float>(), t, times[3], d);
         // The layers (qwen3_asr.rs:344-368): attention within windows.
         for (int l = 0; l < c.layers; ++l) {
-            hipLaunchKernelGGL(layer_norm_kernel, dim3(t), dim3(64), 0, s, x.as<float>(), d, e.norm(l, 0),
-                               e.norm(l, 1), NORM_EPS, xn.as<float>());
+            layer_norm(x.as<float>(), t, d, e.norm(l, 0), e.norm(l, 1), NORM_EPS, xn.as<float>(), s);
             encoder_product(*e.layers[4 * l], xn.as<float>(), t, qkv.as<float>(), nullptr, scratch, s);
             exact_attention_windows(qkv.as<float>(), 3 * d, qkv.as<float>() + d, qkv.as<float>() + 2 * d, 3 * d, t,
                                     window, c.heads, hd, att.as<float>(), kc.as<float>(), vc.as<float>(),
                                     st.as<State>(), s);
             encoder_product(*e.layers[4 * l + 1], att.as<float>(), t, x.as<float>(), x.as<float>(), scratch, s);
-            hipLaunchKernelGGL(layer_norm_kernel, dim3(t), dim3(64), 0, s, x.as<float>(), d, e.norm(l, 2),
-                               e.norm(l, 3), NORM_EPS, xn.as<float>());
+            layer_norm(x.as<float>(), t, d, e.norm(l, 2), e.norm(l, 3), NORM_EPS, xn.as<float>(), s);
             encoder_product(*e.layers[4 * l + 2], xn.as<float>(), t, hid.as<float>(), nullptr, scratch, s);
             hipLaunchKernelGGL(gelu_kernel, dim3(blocks_for((size_t)t * c.ffn)), dim3(256), 0, s, hid.as<float>(),
                                (size_t)t * c.ffn);
             encoder_product(*e.layers[4 * l + 3], hid.as<float>(), t, x.as<float>(), x.as<float>(), scratch, s);
         }
         // ln_post, proj1, GELU, proj2 (qwen3_asr.rs:369-372).
-        hipLaunchKernelGGL(layer_norm_kernel, dim3(t), dim3(64), 0, s, x.as<float>(), d, e.norm(c.layers, 0),
-                           e.norm(c.layers, 1), NORM_EPS, xn.as<float>());
+        layer_norm(x.as<float>(), t, d, e.norm(c.layers, 0), e.norm(c.layers, 1), NORM_EPS, xn.as<float>(), s);
         encoder_product(*e.proj1, xn.as<float>(), t, att.as<float>(), nullptr, scratch, s);
         hipLaunchKernelGGL(gelu_kernel, dim3(blocks_for((size_t)t * d)), dim3(256), 0, s, att.as<float>(),
                            (size_t)t * d);
