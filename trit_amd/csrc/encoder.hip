@@ -290,22 +290,40 @@ using namespace trit;
 
 namespace {
 
-// x W^T (+ bias) of m rows into y (+ residual): the matrix cores for more
-// than 8 rows where the layer allows it, else launches of up to 8 rows.
-void encoder_product(const Layer& L, const float* x, int m, float* y, const float* residual, DeviceMemory& scratch,
-                     hipStream_t s) {
+// Whether a convolution's product over m rows quantizes them straight from
+// its input maps.
+bool quantized_from_maps(const Layer& L, int m, const ConvInput& conv) {
+    GemvArgs a;
+    a.m = m;
+    return m > 8 && gemm_supported(L, a) && gemm_conv_supported(L, conv);
+}
+
+// x W^T (+ bias) of m rows into y: then the GELU, then + residual. The
+// matrix cores for more than 8 rows, the GELU and the add in their store;
+// else launches of up to 8 rows. conv: the rows are a convolution's im2col
+// columns (ConvInput; its maps are `maps`), which take the place of x --
+// quantized from the maps where the layer allows it, else written to x.
+void encoder_product(const Layer& L, float* x, int m, float* y, const float* residual, bool gelu,
+                     DeviceMemory& scratch, hipStream_t s, const ConvInput* conv = nullptr, int maps = 0) {
     GemvArgs a;
     a.x = x;
     a.y = y;
     a.m = m;
+    a.gelu = gelu;
     if (residual) {
         a.residual = residual;
         a.epilogue = EPI_RESIDUAL;
     }
-    if (m > 8 && gemm_supported(L, a)) {
+    const bool whole = m > 8 && gemm_supported(L, a);
+    if (conv && !quantized_from_maps(L, m, *conv)) {
+        hipLaunchKernelGGL(conv2d_columns_kernel, dim3(blocks_for((size_t)m * L.k)), dim3(256), 0, s, conv->in, maps,
+                           conv->bins, conv->times, conv->channels, x);
+        conv = nullptr;
+    }
+    if (whole) {
         const size_t need = gemm_scratch_bytes(m, L.k);
         if (scratch.bytes < need) scratch.alloc(need);
-        return gemm_int(L, a, scratch.ptr, s);
+        return gemm_int(L, a, scratch.ptr, s, conv);
     }
     if (m > 8 && gemm_float_supported(L, a)) return gemm_float(L, a, s);
     if (m > 8 && gemm_float_mfma_supported(L, a)) {
@@ -319,14 +337,24 @@ void encoder_product(const Layer& L, const float* x, int m, float* y, const floa
         a.scratch = scratch.ptr;
         a.scratch_bytes = scratch.bytes;
     }
+    // (A GELU's residual is added after it, below.)
+    a.gelu = 0;
+    if (gelu) {
+        a.residual = nullptr;
+        a.epilogue = EPI_STORE;
+    }
     for (int r0 = 0; r0 < m; r0 += 8) {
         GemvArgs b = a;
         b.m = m - r0 < 8 ? m - r0 : 8;
         b.x = x + (size_t)r0 * L.k;
         b.y = y + (size_t)r0 * L.n;
-        if (residual) b.residual = residual + (size_t)r0 * L.n;
+        if (a.residual) b.residual = residual + (size_t)r0 * L.n;
         layer_forward(L, b, s);
     }
+    const size_t total = (size_t)m * L.n;
+    if (gelu) hipLaunchKernelGGL(gelu_kernel, dim3(blocks_for(total)), dim3(256), 0, s, y, total);
+    if (gelu && residual)
+        hipLaunchKernelGGL(add_kernel, dim3(blocks_for(total)), dim3(256), 0, s, y, residual, total);
 }
 
 // sinusoids (src/layers.rs:257-270): row p is [sin | cos] of (first + p)
@@ -449,17 +477,11 @@ int trit_hip_encoder_encode(const TritHipEncoder* encoder, const float* mel, flo
         size_t n = (size_t)frames * c.mels * 3;
         hipLaunchKernelGGL(im2col_kernel, dim3(blocks_for(n)), dim3(256), 0, s, dmel.as<float>(), frames, c.mels, 3, 1,
                            1, frames, cols.as<float>());
-        encoder_product(*e.conv1, cols.as<float>(), frames, h.as<float>(), nullptr, scratch, s);
-        hipLaunchKernelGGL(gelu_kernel, dim3(blocks_for((size_t)frames * d)), dim3(256), 0, s, h.as<float>(),
-                           (size_t)frames * d);
+        encoder_product(*e.conv1, cols.as<float>(), frames, h.as<float>(), nullptr, true, scratch, s);
         n = (size_t)P * d * 3;
         hipLaunchKernelGGL(im2col_kernel, dim3(blocks_for(n)), dim3(256), 0, s, h.as<float>(), frames, d, 3, 2, 1, P,
                            cols.as<float>());
-        encoder_product(*e.conv2, cols.as<float>(), P, x.as<float>(), nullptr, scratch, s);
-        hipLaunchKernelGGL(gelu_kernel, dim3(blocks_for((size_t)P * d)), dim3(256), 0, s, x.as<float>(),
-                           (size_t)P * d);
-        hipLaunchKernelGGL(add_kernel, dim3(blocks_for((size_t)P * d)), dim3(256), 0, s, x.as<float>(),
-                           e.positions.as<float>(), (size_t)P * d);
+        encoder_product(*e.conv2, cols.as<float>(), P, x.as<float>(), e.positions.as<float>(), true, scratch, s);
         // The layers (audio_encoder.rs:124-136).
         for (int l = 0; l < c.layers; ++l) {
             const Layer& Lqkv = *e.layers[4 * l];
@@ -467,15 +489,13 @@ int trit_hip_encoder_encode(const TritHipEncoder* encoder, const float* mel, flo
             const Layer& Lfc1 = *e.layers[4 * l + 2];
             const Layer& Lfc2 = *e.layers[4 * l + 3];
             layer_norm(x.as<float>(), P, d, e.norm(l, 0), e.norm(l, 1), NORM_EPS, xn.as<float>(), s);
-            encoder_product(Lqkv, xn.as<float>(), P, qkv.as<float>(), nullptr, scratch, s);
+            encoder_product(Lqkv, xn.as<float>(), P, qkv.as<float>(), nullptr, false, scratch, s);
             exact_attention(qkv.as<float>(), 3 * d, qkv.as<float>() + d, qkv.as<float>() + 2 * d, 3 * d, P, P, c.heads,
                             c.heads, hd, 0, att.as<float>(), kc.as<float>(), vc.as<float>(), st.as<State>(), s);
-            encoder_product(Lout, att.as<float>(), P, x.as<float>(), x.as<float>(), scratch, s);
+            encoder_product(Lout, att.as<float>(), P, x.as<float>(), x.as<float>(), false, scratch, s);
             layer_norm(x.as<float>(), P, d, e.norm(l, 2), e.norm(l, 3), NORM_EPS, xn.as<float>(), s);
-            encoder_product(Lfc1, xn.as<float>(), P, hid.as<float>(), nullptr, scratch, s);
-            hipLaunchKernelGGL(gelu_kernel, dim3(blocks_for((size_t)P * c.ffn)), dim3(256), 0, s, hid.as<float>(),
-                               (size_t)P * c.ffn);
-            encoder_product(Lfc2, hid.as<float>(), P, x.as<float>(), x.as<float>(), scratch, s);
+            encoder_product(Lfc1, xn.as<float>(), P, hid.as<float>(), nullptr, true, scratch, s);
+            encoder_product(Lfc2, hid.as<float>(), P, x.as<float>(), x.as<float>(), false, scratch, s);
         }
         layer_norm(x.as<float>(), P, d, e.norm(c.layers, 0), e.norm(c.layers, 1), NORM_EPS, xn.as<float>(), s);
         TRIT_HIP(hipGetLastError());
@@ -570,7 +590,9 @@ int trit_hip_asr_encoder_encode(const TritHipAsrEncoder* encoder, const float* m
         size_t col_floats = (size_t)t * ch * bins[3], map_floats = (size_t)maps * c.mels * longest;
         for (int i = 1; i < 4; ++i) {
             const size_t positions = (size_t)maps * bins[i] * times[i];
-            col_floats = std::max(col_floats, positions * (i == 1 ? 9 : 9 * ch));
+            const ConvInput conv{nullptr, bins[i - 1], times[i - 1], i == 1 ? 1 : ch};
+            if (!quantized_from_maps(*e.convs[i - 1], (int)positions, conv))
+                col_floats = std::max(col_floats, positions * 9 * conv.channels);
             map_floats = std::max(map_floats, positions * ch);
         }
         std::lock_guard<std::mutex> lock(e.ws.mu);
@@ -598,37 +620,32 @@ int trit_hip_asr_encoder_encode(const TritHipAsrEncoder* encoder, const float* m
         for (int i = 0; i < 3; ++i) {
             const int cin = i == 0 ? 1 : ch;
             const size_t rows = (size_t)maps * bins[i + 1] * times[i + 1];
-            hipLaunchKernelGGL(conv2d_columns_kernel, dim3(blocks_for(rows * cin * 9)), dim3(256), 0, s,
-                               map.as<float>(), maps, bins[i], times[i], cin, cols.as<float>());
-            encoder_product(*e.convs[i], cols.as<float>(), (int)rows, map.as<float>(), nullptr, scratch, s);
-            hipLaunchKernelGGL(gelu_kernel, dim3(blocks_for(rows * ch)), dim3(256), 0, s, map.as<float>(),
-                               rows * ch);
+            // (The columns are read off the maps before the product overwrites them.)
+            const ConvInput conv{map.as<float>(), bins[i], times[i], cin};
+            encoder_product(*e.convs[i], cols.as<float>(), (int)rows, map.as<float>(), nullptr, true, scratch, s, &conv,
+                            maps);
         }
         hipLaunchKernelGGL(time_columns_kernel, dim3(blocks_for((size_t)t * ch * bins[3])), dim3(256), 0, s,
                            map.as<float>(), bins[3], times[3], ch, t, cols.as<float>());
-        encoder_product(*e.conv_out, cols.as<float>(), t, x.as<float>(), nullptr, scratch, s);
+        encoder_product(*e.conv_out, cols.as<float>(), t, x.as<float>(), nullptr, false, scratch, s);
         hipLaunchKernelGGL(add_positions_kernel, dim3(blocks_for((size_t)t * d)), dim3(256), 0, s, x.as<float>(),
                            e.positions.as<float>(), t, times[3], d);
         // The layers (qwen3_asr.rs:344-368): attention within windows.
         for (int l = 0; l < c.layers; ++l) {
             layer_norm(x.as<float>(), t, d, e.norm(l, 0), e.norm(l, 1), NORM_EPS, xn.as<float>(), s);
-            encoder_product(*e.layers[4 * l], xn.as<float>(), t, qkv.as<float>(), nullptr, scratch, s);
+            encoder_product(*e.layers[4 * l], xn.as<float>(), t, qkv.as<float>(), nullptr, false, scratch, s);
             exact_attention_windows(qkv.as<float>(), 3 * d, qkv.as<float>() + d, qkv.as<float>() + 2 * d, 3 * d, t,
                                     window, c.heads, hd, att.as<float>(), kc.as<float>(), vc.as<float>(),
                                     st.as<State>(), s);
-            encoder_product(*e.layers[4 * l + 1], att.as<float>(), t, x.as<float>(), x.as<float>(), scratch, s);
+            encoder_product(*e.layers[4 * l + 1], att.as<float>(), t, x.as<float>(), x.as<float>(), false, scratch, s);
             layer_norm(x.as<float>(), t, d, e.norm(l, 2), e.norm(l, 3), NORM_EPS, xn.as<float>(), s);
-            encoder_product(*e.layers[4 * l + 2], xn.as<float>(), t, hid.as<float>(), nullptr, scratch, s);
-            hipLaunchKernelGGL(gelu_kernel, dim3(blocks_for((size_t)t * c.ffn)), dim3(256), 0, s, hid.as<float>(),
-                               (size_t)t * c.ffn);
-            encoder_product(*e.layers[4 * l + 3], hid.as<float>(), t, x.as<float>(), x.as<float>(), scratch, s);
+            encoder_product(*e.layers[4 * l + 2], xn.as<float>(), t, hid.as<float>(), nullptr, true, scratch, s);
+            encoder_product(*e.layers[4 * l + 3], hid.as<float>(), t, x.as<float>(), x.as<float>(), false, scratch, s);
         }
         // ln_post, proj1, GELU, proj2 (qwen3_asr.rs:369-372).
         layer_norm(x.as<float>(), t, d, e.norm(c.layers, 0), e.norm(c.layers, 1), NORM_EPS, xn.as<float>(), s);
-        encoder_product(*e.proj1, xn.as<float>(), t, att.as<float>(), nullptr, scratch, s);
-        hipLaunchKernelGGL(gelu_kernel, dim3(blocks_for((size_t)t * d)), dim3(256), 0, s, att.as<float>(),
-                           (size_t)t * d);
-        encoder_product(*e.proj2, att.as<float>(), t, hid.as<float>(), nullptr, scratch, s);
+        encoder_product(*e.proj1, xn.as<float>(), t, att.as<float>(), nullptr, true, scratch, s);
+        encoder_product(*e.proj2, att.as<float>(), t, hid.as<float>(), nullptr, false, scratch, s);
         TRIT_HIP(hipGetLastError());
         TRIT_HIP(hipMemcpyAsync(out, hid.ptr, (size_t)t * c.out * 4, hipMemcpyDeviceToHost, s));
         TRIT_HIP(hipStreamSynchronize(s));

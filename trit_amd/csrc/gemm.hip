@@ -122,6 +122,73 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__
     if (live && col % G == 0) xs[(size_t)(col / G) * mpad + row] = real ? (HALF ? f16_round(scale) : scale) : 0.0f;
 }
 
+// The same over the im2col rows of a kernel-3, stride-2, padding-1 2-D
+// convolution, from its [map][bin][time][channel] input: column c * 9 + tap of
+// a row is tap's pixel's channel c, zero outside the map
+// (src/models/families/qwen3_asr.rs:408-428). A row's nine pixels go to LDS
+// (each a run of channels; the pitch of 15 mod 32 floats spreads the taps over
+// the banks), the groups are read from there in column order, so the columns
+// never reach memory in f32: with them written and read back, the 24000 rows
+// of 4320 columns that 30 s of audio make took 250 us + 150 us. An XCD takes
+// consecutive rows, which share pixels.
+constexpr int CONV_ROWS = 4;  // rows a block
+
+__host__ __device__ constexpr int conv_pitch(int channels) { return (channels + 16) / 32 * 32 + 15; }
+
+template <int G, bool HALF>
+__global__ __launch_bounds__(256) void quantize_conv_kernel(ConvInput in, int m, int mpad, int8_t* __restrict__ xq,
+                                                            float* __restrict__ xs, const int* skip) {
+    if (skip && *skip) return;
+    extern __shared__ float px[];  // [tap][pitch]
+    constexpr int TPG = G / 4;
+    const int ch = in.channels, pitch = conv_pitch(ch), k = 9 * ch;
+    const int ob = (in.bins + 1) / 2, ot = (in.times + 1) / 2;
+    const int id = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
+    for (int row = id * CONV_ROWS; row < min((id + 1) * CONV_ROWS, mpad); ++row) {
+        if (row >= m) {
+            for (int g = threadIdx.x; g < k / G; g += 256) xs[(size_t)g * mpad + row] = 0.0f;
+            continue;
+        }
+        const int xo = row % ot, yo = row / ot % ob, map = row / (ot * ob);
+        __syncthreads();  // the row before is read
+        for (int i = threadIdx.x; i < 9 * (ch / 4); i += 256) {
+            const int tap = i / (ch / 4), c = (i - tap * (ch / 4)) * 4;
+            const int sy = 2 * yo + tap / 3 - 1, sx = 2 * xo + tap % 3 - 1;
+            float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (sy >= 0 && sy < in.bins && sx >= 0 && sx < in.times)
+                v = *(const float4*)(in.in + (((size_t)map * in.bins + sy) * in.times + sx) * ch + c);
+            float* to = px + tap * pitch + c;
+            to[0] = v.x;
+            to[1] = v.y;
+            to[2] = v.z;
+            to[3] = v.w;
+        }
+        __syncthreads();
+        // k / 4 is a multiple of TPG, so a group's lanes take an item together.
+        for (int i = threadIdx.x; i < k / 4; i += 256) {
+            float v[4];
+            int c = 4 * i / 9, tap = 4 * i - 9 * c;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                v[u] = px[tap * pitch + c];
+                if (++tap == 9) {
+                    tap = 0;
+                    ++c;
+                }
+            }
+            float peak = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(v[0]), __builtin_fabsf(v[1])),
+                                         __builtin_fmaxf(__builtin_fabsf(v[2]), __builtin_fabsf(v[3])));
+#pragma unroll
+            for (int off = TPG / 2; off > 0; off >>= 1) peak = __builtin_fmaxf(peak, __shfl_xor(peak, off));
+            const float scale = peak > 0.0f ? peak / 127.0f : 1.0f;
+            const float q = 1.0f / scale;
+            *(uint32_t*)(xq + (size_t)row * k + 4 * i) =
+                pack4(act_code(v[0] * q), act_code(v[1] * q), act_code(v[2] * q), act_code(v[3] * q));
+            if (4 * i % G == 0) xs[(size_t)(4 * i / G) * mpad + row] = HALF ? f16_round(scale) : scale;
+        }
+    }
+}
+
 constexpr int KC = 256;           // bytes of K per LDS chunk
 constexpr int ROW_LDS = KC + 16;  // padded LDS row: rows 8 apart start 4 banks apart
 constexpr int BN_ROWS = 128;      // weight rows per block
@@ -387,6 +454,10 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(const int8_t* __r
             v0 = __builtin_fmaxf(v0, 0.0f);
             v1 = __builtin_fmaxf(v1, 0.0f);
         }
+        if (P == 1 && a.gelu) {
+            v0 = gelu_trit(v0);
+            v1 = gelu_trit(v1);
+        }
         if (P == 2) {
             a.y[(size_t)row * ldy + r0 + lr] = silu_trit(v0) * v1;
             continue;
@@ -649,6 +720,10 @@ __global__ __launch_bounds__(GEMM_THREADS, TW == 2 ? 3 : 4) void gemm_dma_kernel
             v0 = __builtin_fmaxf(v0, 0.0f);
             v1 = __builtin_fmaxf(v1, 0.0f);
         }
+        if (P == 1 && a.gelu) {
+            v0 = gelu_trit(v0);
+            v1 = gelu_trit(v1);
+        }
         if (P == 2) {
             a.y[(size_t)row * ldy + r0 + lr] = silu_trit(v0) * v1;
             continue;
@@ -768,6 +843,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_ternary_kernel(const int
             float v = t[j][r];
             if (bias) v = v + bias[col];
             if (a.relu) v = __builtin_fmaxf(v, 0.0f);
+            if (a.gelu) v = gelu_trit(v);
             const size_t at = (size_t)row * n + col;
             a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v : v;
         }
@@ -874,7 +950,12 @@ size_t gemm_scratch_bytes(int m, int k) {
     return al((size_t)m * k) + al((size_t)(k / 32) * mpad * 4) + al(mpad * 4);
 }
 
-void gemm_int(const Layer& L, const GemvArgs& a, void* scratch, hipStream_t s) {
+bool gemm_conv_supported(const Layer& L, const ConvInput& in) {
+    return !float_kind(L.kind) && L.k == 9 * in.channels && in.channels % 4 == 0 &&
+           (size_t)9 * conv_pitch(in.channels) * 4 <= 64 * 1024;
+}
+
+void gemm_int(const Layer& L, const GemvArgs& a, void* scratch, hipStream_t s, const ConvInput* conv) {
     if (!gemm_supported(L, a)) fail("gemm: layer " + std::to_string(L.n) + "x" + std::to_string(L.k) +
                                     " is not a shape the matrix-core product takes");
     const Scratch sc = carve(scratch, a.m, L.k);
@@ -887,7 +968,17 @@ void gemm_int(const Layer& L, const GemvArgs& a, void* scratch, hipStream_t s) {
     const int G = group_of(L);
     const size_t items = (size_t)sc.mpad * (L.k / 4);
     const int qblocks = (int)((items + 255) / 256);
-    if (G == 32)
+    if (conv) {
+        if (!gemm_conv_supported(L, *conv) || a.norm_w) fail("gemm: not a convolution the quantizer takes");
+        const size_t lds = (size_t)9 * conv_pitch(conv->channels) * 4;
+        const int blocks = (sc.mpad / CONV_ROWS + 7) / 8 * 8;
+        if (G == 32)
+            hipLaunchKernelGGL((quantize_conv_kernel<32, true>), dim3(blocks), dim3(256), lds, s, *conv, a.m, sc.mpad,
+                               sc.xq, sc.xs, a.skip);
+        else
+            hipLaunchKernelGGL((quantize_conv_kernel<128, false>), dim3(blocks), dim3(256), lds, s, *conv, a.m,
+                               sc.mpad, sc.xq, sc.xs, a.skip);
+    } else if (G == 32)
         hipLaunchKernelGGL((quantize_kernel<32, true>), dim3(qblocks), dim3(256), 0, s, a.x, a.m, sc.mpad, L.k,
                            a.norm_w, inv, sc.xq, sc.xs, a.skip);
     else

@@ -262,6 +262,7 @@ __global__ __launch_bounds__(THREADS, 2) void float_mfma_kernel(const float4* __
         float v = (part[0][e] + part[2][e]) + (part[1][e] + part[3][e]);
         if (bias) v = v + bias[col];
         if (a.relu) v = __builtin_fmaxf(v, 0.0f);
+        if (a.gelu) v = gelu_trit(v);
         const size_t at = (size_t)row * n + col;
         a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v : v;
     }

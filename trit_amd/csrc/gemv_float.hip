@@ -332,8 +332,16 @@ __global__ __launch_bounds__(THREADS) void float_rows_kernel(const typename WT<K
         float h[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) h[i] = l[i] + l[i + 8];
-        const float v = ((h[0] + h[4]) + (h[2] + h[6])) + ((h[1] + h[5]) + (h[3] + h[7]));
-        store_out(a, bias, n, f, col, v);
+        float v = ((h[0] + h[4]) + (h[2] + h[6])) + ((h[1] + h[5]) + (h[3] + h[7]));
+        if (a.gelu) {
+            if (bias) v = v + bias[col];
+            if (a.relu) v = __builtin_fmaxf(v, 0.0f);
+            const size_t at = (size_t)f * n + col;
+            v = gelu_trit(v);
+            a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v : v;
+        } else {
+            store_out(a, bias, n, f, col, v);
+        }
     }
 }
 

@@ -135,6 +135,9 @@ struct GemvArgs {
     const float* residual = nullptr;
     int epilogue = EPI_STORE;
     int relu = 0;
+    // The exact GELU on the output, before the residual add (the products of
+    // many rows only: gemm_int without the pair, gemm_float, gemm_float_mfma).
+    int gelu = 0;
     // Device flag: nonzero skips the launch (a finished decode loop).
     const int* skip = nullptr;
     // Measurement: events stamped at the product kernel's start and end
@@ -211,7 +214,15 @@ void gemm_float_mfma(const Layer& L, GemvArgs a, void* scratch, size_t scratch_b
 // device memory the product may overwrite.
 bool gemm_supported(const Layer& L, const GemvArgs& a);
 size_t gemm_scratch_bytes(int m, int k);
-void gemm_int(const Layer& L, const GemvArgs& a, void* scratch, hipStream_t s);
+// conv: the rows are the im2col columns of a kernel-3, stride-2, padding-1
+// convolution of maps [bin][time][channel] (k = 9 * channels), quantized
+// straight from them; a.x is not read.
+struct ConvInput {
+    const float* in;
+    int bins, times, channels;
+};
+bool gemm_conv_supported(const Layer& L, const ConvInput& in);
+void gemm_int(const Layer& L, const GemvArgs& a, void* scratch, hipStream_t s, const ConvInput* conv = nullptr);
 // Any layer kind.
 void layer_forward(const Layer& L, const GemvArgs& a, hipStream_t s);
 
