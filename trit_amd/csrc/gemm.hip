@@ -601,7 +601,6 @@ __global__ __launch_bounds__(GEMM_THREADS, TW == 2 ? 3 : 4) void gemm_dma_kernel
     const int wn = w / 2;
     const int sub0 = TW == 1 ? wn * 32 : P == 1 ? wn * 64 : wn * 32;
     const int sub1 = TW == 1 ? sub0 : P == 1 ? wn * 64 + 32 : 64 + wn * 32;
-    const int xrow = (w % 2) * 32 + 4 * h;
     uint32_t pa[4], pb[4];
 #pragma unroll
     for (int s4 = 0; s4 < 4; ++s4) {
@@ -615,65 +614,74 @@ __global__ __launch_bounds__(GEMM_THREADS, TW == 2 ? 3 : 4) void gemm_dma_kernel
 #pragma unroll
     for (int r = 0; r < 16; ++r) t0[r] = t1[r] = 0.0f;
 
+    // The scale products come from the matrix cores: the outer product of 32 x
+    // scales and 32 weight scales in the dots' register layout, each
+    // fma(xs, ws, 0), which is the vector multiply's one rounding.
+    // v_mfma_f32_32x32x1_2b makes two of them, of a tile's two groups (TW = 1)
+    // or of the two tiles (TW = 2), half h of the lanes giving the second's
+    // scales. LDS bounded the kernel (busy 94% of its time), two thirds of it
+    // the sixteen x scales a lane read for the multiply; the outer product
+    // reads one. The conversions of two tiles go before their multiply-adds:
+    // a dependent vector instruction costs 10.5 cycles, and without the
+    // scheduling barriers the compiler pairs each multiply-add with the
+    // conversion just before it (in that order the outer product was slower
+    // than the multiply: 55 us a 1564-row product against 46). The three
+    // products of a 1564-row prompt (n 2048, 6144, 2048; k 2048): 139 -> 126 us.
+    const v16i magic = dot_base();
+    const int xr = (w % 2) * 32 + lr, wr = TW == 1 ? sub0 + lr : (h ? sub1 : sub0) + lr;
+    auto weight_scale = [&](const DStage<TW>& s, int g) {
+        if (HALF) return f16_to_f32(((const uint16_t*)s.ws)[4 * wr + g]);
+        return __builtin_bit_cast(float, s.ws[wr]);
+    };
     auto compute = [&](const DStage<TW>& s) {
         const int8_t* sa = s.a;
         const int8_t* sb = s.b;
-        // The stage's weight scales of the lane's columns.
-        float wsc0[GPC], wsc1[GPC];
-        if (HALF) {
-            const uint2 u0 = *(const uint2*)(s.ws + 2 * (sub0 + lr));
-            const uint2 u1 = TW == 2 ? *(const uint2*)(s.ws + 2 * (sub1 + lr)) : u0;
-            const uint32_t v0[2] = {u0.x, u0.y}, v1[2] = {u1.x, u1.y};
-#pragma unroll
-            for (int g = 0; g < GPC; ++g) {
-                wsc0[g] = f16_to_f32((uint16_t)(v0[g / 2] >> (16 * (g % 2))));
-                wsc1[g] = f16_to_f32((uint16_t)(v1[g / 2] >> (16 * (g % 2))));
-            }
-        } else {
-            wsc0[0] = __builtin_bit_cast(float, s.ws[sub0 + lr]);
-            wsc1[0] = __builtin_bit_cast(float, s.ws[sub1 + lr]);
-        }
-        Frags<CH> f;
-#pragma unroll
-        for (int c4 = 0; c4 < CH; ++c4) {
-            f.a[c4] = *(const v4i*)(sa + pa[c4]);
-            f.b0[c4] = *(const v4i*)(sb + pb[c4]);
-            if (TW == 2) f.b1[c4] = *(const v4i*)(sb + pb[c4] + B1);
-        }
-#pragma unroll
-        for (int gi = 0; gi < GPC; ++gi) {
-            v16i d0 = {}, d1 = {};
+        auto dots = [&](int g, int tile) {
+            v16i d = magic;
 #pragma unroll
             for (int c4 = 0; c4 < CH; ++c4) {
-                d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[c4], f.b0[c4], d0, 0, 0, 0);
-                if (TW == 2) d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[c4], f.b1[c4], d1, 0, 0, 0);
+                const int s4 = g * CH + c4;
+                d = __builtin_amdgcn_mfma_i32_32x32x32_i8(*(const v4i*)(sa + pa[s4]),
+                                                          *(const v4i*)(sb + pb[s4] + tile * B1), d, 0, 0, 0);
             }
+            return d;
+        };
+        // Two dots' chain steps: all the conversions, then the multiply-adds.
+        auto chain2 = [&](float (&ta)[16], float (&tb)[16], const v16i& d0, const v16i& d1, const v32f& sc) {
+            float f0[16], f1[16];
             __builtin_amdgcn_sched_barrier(0);
-            if (gi + 1 < GPC) {
 #pragma unroll
-                for (int c4 = 0; c4 < CH; ++c4) {
-                    const int s4 = (gi + 1) * CH + c4;
-                    f.a[c4] = *(const v4i*)(sa + pa[s4]);
-                    f.b0[c4] = *(const v4i*)(sb + pb[s4]);
-                    if (TW == 2) f.b1[c4] = *(const v4i*)(sb + pb[s4] + B1);
-                }
+            for (int r = 0; r < 16; ++r) f0[r] = dot_of(d0[r]);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) f1[r] = dot_of(d1[r]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) ta[r] = __builtin_fmaf(f0[r], sc[r], ta[r]);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) tb[r] = __builtin_fmaf(f1[r], sc[16 + r], tb[r]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if constexpr (TW == 2) {
+#pragma unroll
+            for (int g = 0; g < GPC; ++g) {
+                const v32f sc = __builtin_amdgcn_mfma_f32_32x32x1f32(s.xs[g * BM + xr], weight_scale(s, g), v32f{}, 0, 0, 0);
+                const v16i d0 = dots(g, 0), d1 = dots(g, 1);
+                chain2(t0, t1, d0, d1, sc);
             }
-            float4 xv4[4];
+        } else if constexpr (GPC > 1) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) xv4[q] = *(const float4*)(s.xs + gi * BM + xrow + 8 * q);
-            __builtin_amdgcn_sched_barrier(0);
-            // Output (row 8*(r/4) + 4h + r%4, column lr) of a tile is register r.
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float xv[4] = {xv4[q].x, xv4[q].y, xv4[q].z, xv4[q].w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int r = 4 * q + j;
-                    t0[r] = __builtin_fmaf((float)d0[r], wsc0[gi] * xv[j], t0[r]);
-                    if (TW == 2) t1[r] = __builtin_fmaf((float)d1[r], wsc1[gi] * xv[j], t1[r]);
-                }
+            for (int g = 0; g < GPC; g += 2) {
+                const v32f sc = __builtin_amdgcn_mfma_f32_32x32x1f32(s.xs[(g + h) * BM + xr], weight_scale(s, g + h), v32f{}, 0, 0, 0);
+                const v16i d0 = dots(g, 0), d1 = dots(g + 1, 0);
+                chain2(t0, t0, d0, d1, sc);
             }
-            __builtin_amdgcn_sched_barrier(0);
+        } else {
+            // One group a stage: the second K step's product is 0 * 0.
+            const float xv = s.xs[xr], wv = weight_scale(s, 0);
+            const v16f sc = __builtin_amdgcn_mfma_f32_32x32x2f32(h ? 0.0f : xv, h ? 0.0f : wv, v16f{}, 0, 0, 0);
+            const v16i d = dots(0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) t0[r] = __builtin_fmaf(dot_of(d[r]), sc[r], t0[r]);
         }
     };
 
