@@ -1,0 +1,26 @@
+"""Q8_0 products large enough for 128 x 128 blocks whose k is not a multiple of
+128, against the oracle, bit for bit: one to thirty-nine groups (odd counts, so
+a row's scales start at either half of a dword), rows and columns past the last
+whole block, bias and relu."""
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from trit_amd import hip, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,k,m", [(20480, 32, 9), (1312, 64, 1900), (96, 160, 20450), (1312, 416, 1921),
+                                   (480, 1248, 5100)])
+def test_wide(gpu, n, k, m):
+    print(f"case q8_0 wide blocks n={n} k={k} m={m}", flush=True)
+    codes, sbits = synth.q8_0_matrix(synth.seed_for(2, n + k), n, k)
+    bias = synth.activations(91, 1, n)[0]
+    x = synth.activations(92 + m, m, k)
+    layer = hip.Dense.q8_0(n, k, synth.q8_0_blocks(codes, sbits), bias)
+    got = layer.forward(x, relu=True)
+    want = np.maximum(O.Int8(codes, sbits.view(np.float16).astype(np.float32), 32, True)(x) + bias, 0)
+    assert np.array_equal(got.view(np.uint32), want.astype(np.float32).view(np.uint32))
+    layer.free()

@@ -742,6 +742,187 @@ __global__ __launch_bounds__(GEMM_THREADS, TW == 2 ? 3 : 4) void gemm_dma_kernel
     }
 }
 
+// Large Q8_0 / Q4_K products of k not a multiple of 128 (an ASR stem's 4320-input
+// convolutions): 128 x rows by 128 weight rows a block, stages as above, two
+// blocks a CU by their LDS (73 KB). A wave owns 64 x 64 outputs as 2 x 2 MFMA
+// tiles, so a byte loaded and a byte read from LDS feed twice the outputs of
+// the 64 x 64 blocks, in half the waves. Scale products and conversions as
+// above. The last stage's pieces past k load the row's first piece of the
+// stage, its groups past k are not chained, and a row's four f16 scales, which
+// start at any 2-byte offset, are loaded as the three dwords that hold them.
+struct alignas(16) WStage {
+    alignas(16) int8_t a[128 * KD];
+    alignas(16) int8_t b[128 * KD];
+    alignas(16) float xs[4 * 128];  // [group of the stage][x row]
+    alignas(16) uint32_t ws[3 * 128];
+};
+
+__global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_wide_kernel(
+    const int8_t* __restrict__ xq, const float* __restrict__ xs, int m, int mpad, const int8_t* __restrict__ codes,
+    const void* __restrict__ scales, const float* __restrict__ bias, int n, int k, int nb, int mb, GemvArgs a) {
+    __shared__ WStage st0, st1;
+    if (a.skip && *a.skip) return;
+    const int groups = k / 32, chunks = (k + KD - 1) / KD;
+    const int blk = blockIdx.x;
+    int bn, bm;
+    if (nb % 8 == 0) {
+        const int q = blk / 8;
+        bn = blk % 8 + 8 * (q / mb);
+        bm = q % mb;
+    } else {
+        bn = blk % nb;
+        bm = blk / nb;
+    }
+    const int t = threadIdx.x;
+    const int lane = t % WAVE, w = __builtin_amdgcn_readfirstlane(t / WAVE);
+    const int lr = lane % 32, h = lane / 32;
+    const int mbase = bm * 128;
+    // LDS weight row i holds weight row brow(i); rows past n load row n - 1.
+    auto brow = [&](int i) { return min(bn * 128 + i, n - 1); };
+
+    // The wave's loads of a stage: x rows and weight rows [32 w, +32), 1 KB
+    // (eight rows of 128 bytes) an instruction; then scale items w and w + 4
+    // (x scales, 16 bytes a lane; weight scales, a dword a lane).
+    uint32_t ag[4], bg[4], piece[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int rl = 8 * (4 * w + i) + lane / 8;
+        piece[i] = 16 * ((lane % 8) ^ piece_swizzle(rl));
+        ag[i] = (uint32_t)(mbase + rl < m ? mbase + rl : m - 1) * (uint32_t)k;
+        bg[i] = (uint32_t)brow(rl) * (uint32_t)k;
+    }
+    // Items 0 and 1 are the x scales of two groups each, 2 .. 7 the weight
+    // rows' scale dwords.
+    int item[2];
+    size_t soff[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        item[j] = w + 4 * j;
+        const int d = 64 * (item[j] - 2) + lane;
+        // x rows past mpad (none of them stored) take its last four.
+        soff[j] = item[j] < 2 ? (size_t)min(mbase + 4 * (lane % 32), mpad - 4)
+                              : ((size_t)brow(d / 3) * groups) / 2 + d % 3;
+    }
+    const size_t last_dword = ((size_t)n * groups - 1) / 2;
+    auto issue = [&](int c, WStage& s) {
+        const size_t off = (size_t)c * KD;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t p = (int)(off + piece[i]) < k ? piece[i] : 0;
+            load16_to_lds(xq + ag[i] + off + p, s.a + 1024 * (4 * w + i));
+            load16_to_lds(codes + bg[i] + off + p, s.b + 1024 * (4 * w + i));
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if (item[j] < 2) {
+                const int g = min(4 * c + 2 * item[j] + lane / 32, groups - 1);
+                load16_to_lds(xs + soff[j] + (size_t)g * mpad, s.xs + 256 * item[j]);
+            } else {
+                load4_to_lds((const uint32_t*)scales + min(soff[j] + 2 * c, last_dword), s.ws + 64 * (item[j] - 2));
+            }
+        }
+    };
+
+    // The wave's tiles: x rows [64 (w % 2), +64) of the block, weight LDS rows
+    // sub0 and sub1, 32 each. Lane (lr, h) reads piece 2 s + h of its rows for
+    // step s; its rows all share (lr >> 1) & 7.
+    const int wn = w / 2;
+    const int sub0 = wn * 64, sub1 = sub0 + 32;
+    const int xr = (w % 2) * 64 + lr, wr = (h ? sub1 : sub0) + lr;
+    uint32_t pa[4], pb[4];
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4) {
+        const int po = 16 * ((2 * s4 + h) ^ piece_swizzle(lr));
+        pa[s4] = xr * KD + po;
+        pb[s4] = (sub0 + lr) * KD + po;
+    }
+    constexpr int T1 = 32 * KD;  // a tile
+    // Half h of the lanes holds the scales of tile h: their first's offset in the three dwords.
+    const int wodd = (int)(((size_t)brow(wr) * groups) & 1);
+    const v16i magic = dot_base();
+    float acc[2][2][16];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+    auto compute = [&](const WStage& s, int c) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if (4 * c + g >= groups) break;
+            const float wv = f16_to_f32(((const uint16_t*)s.ws)[6 * wr + wodd + g]);
+            const v4i fa[2] = {*(const v4i*)(s.a + pa[g]), *(const v4i*)(s.a + pa[g] + T1)};
+            const v4i fb[2] = {*(const v4i*)(s.b + pb[g]), *(const v4i*)(s.b + pb[g] + T1)};
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const v32f sc = __builtin_amdgcn_mfma_f32_32x32x1f32(s.xs[g * 128 + xr + 32 * i], wv, v32f{}, 0, 0, 0);
+                v16i d[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) d[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], magic, 0, 0, 0);
+                // Output (row 8*(r/4) + 4h + r%4, column lr) of a tile is register r.
+                // Conversions first, as in the kernel above.
+                float f[2][16];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) f[j][r] = dot_of(d[j][r]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        acc[i][j][r] = __builtin_fmaf(f[j][r], sc[16 * j + r], acc[i][j][r]);
+            }
+        }
+    };
+
+    // Two stages: stage c + 1 loads while stage c computes.
+    auto step = [&](int c, WStage& cur, WStage& next) {
+        // This wave's loads of stage c (the only ones in flight) landed; the
+        // barrier: every wave's, and every wave is done with stage c - 1,
+        // whose buffer stage c + 1 takes.
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+        asm volatile("s_barrier" ::: "memory");
+        if (c + 1 < chunks) issue(c + 1, next);
+        compute(cur, c);
+    };
+    issue(0, st0);
+    for (int c = 0; c < chunks; c += 2) {
+        step(c, st0, st1);
+        if (c + 1 >= chunks) break;
+        step(c + 1, st1, st0);
+    }
+
+    // Epilogue, as gemm_kernel's (src/models/parts/causal_lm.rs:464-473).
+    const int r0 = bn * 128 + sub0, r1 = r0 + 32;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = mbase + (w % 2) * 64 + 32 * i + 8 * (r / 4) + 4 * h + r % 4;
+            if (row >= m) continue;
+            float v0 = acc[i][0][r], v1 = acc[i][1][r];
+            if (bias) {
+                v0 = v0 + bias[min(r0 + lr, n - 1)];
+                v1 = v1 + bias[min(r1 + lr, n - 1)];
+            }
+            if (a.relu) {
+                v0 = __builtin_fmaxf(v0, 0.0f);
+                v1 = __builtin_fmaxf(v1, 0.0f);
+            }
+            if (a.gelu) {
+                v0 = gelu_trit(v0);
+                v1 = gelu_trit(v1);
+            }
+            const size_t i0 = (size_t)row * n + r0 + lr, i1 = (size_t)row * n + r1 + lr;
+            if (r0 + lr < n) a.y[i0] = a.epilogue == EPI_RESIDUAL ? a.residual[i0] + v0 : v0;
+            if (r1 + lr < n) a.y[i1] = a.epilogue == EPI_RESIDUAL ? a.residual[i1] + v1 : v1;
+        }
+}
+
 // Ternary products of many rows: 2-bit codes, f32 scales a 128-group, the
 // same contract (dot of the codes minus one and the activation codes). A wave
 // owns 32 x rows by TN 32-row weight tiles, four waves a block (2 x 2); no LDS
@@ -892,10 +1073,27 @@ bool narrow(int n, int mb) {
     return true;
 }
 
+// Whether a plain product takes gemm_wide_kernel: k not a multiple of 128, and
+// 128 x 128 blocks for most CUs (n 480, k 4320, with the GELU: 24000 rows, 752
+// blocks, 218 us against 337 us for gemm_kernel; 6000 rows, 196 blocks, 95 us
+// against 111). For other k the 64 x 64 blocks are faster (1564 x 6144 x 2048,
+// 624 blocks: 68 us against 82).
+bool wide(int nb, int m, int k) { return k % KD != 0 && (int64_t)nb * ((m + 127) / 128) >= 160; }
+
 template <int G, bool HALF, int P>
 void launch_gemm(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStream_t s) {
     const int nb = P == 1 ? (L.n + 127) / 128 : (L.n / 2) / 64;
     const int mb = sc.mpad / BM;
+    if constexpr (G == 32 && P == 1) {
+        if (wide(nb, a.m, L.k)) {
+            const int mb2 = (a.m + 127) / 128;
+            launch_timed(a, gemm_wide_kernel, dim3(nb * mb2), dim3(GEMM_THREADS), 0, s, (const int8_t*)sc.xq,
+                         (const float*)sc.xs, a.m, sc.mpad, L.codes.as<int8_t>(), (const void*)L.scales.ptr,
+                         L.bias.as<float>(), L.n, L.k, nb, mb2, a);
+            TRIT_HIP(hipGetLastError());
+            return;
+        }
+    }
     if constexpr (P == 1) {
         if (L.k % KD == 0 && narrow(L.n, mb)) {
             const int nb1 = (L.n + 63) / 64;
@@ -910,11 +1108,7 @@ void launch_gemm(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStream
         launch_timed(a, gemm_dma_kernel<G, HALF, P, 2>, dim3(nb * mb), dim3(GEMM_THREADS), 0, s,
                      (const int8_t*)sc.xq, (const float*)sc.xs, a.m, sc.mpad, L.codes.as<int8_t>(),
                      (const void*)L.scales.ptr, L.bias.as<float>(), L.n, L.k, nb, mb, a);
-    else if (L.k % KC == 0)
-        launch_timed(a, gemm_kernel<G, HALF, P, false>, dim3(nb * mb), dim3(GEMM_THREADS), 0, s,
-                     (const int8_t*)sc.xq, (const float*)sc.xs, a.m, sc.mpad, L.codes.as<int8_t>(),
-                     (const void*)L.scales.ptr, L.bias.as<float>(), L.n, L.k, nb, mb, a);
-    else
+    else if constexpr (G == 32)
         launch_timed(a, gemm_kernel<G, HALF, P, true>, dim3(nb * mb), dim3(GEMM_THREADS), 0, s,
                      (const int8_t*)sc.xq, (const float*)sc.xs, a.m, sc.mpad, L.codes.as<int8_t>(),
                      (const void*)L.scales.ptr, L.bias.as<float>(), L.n, L.k, nb, mb, a);
