@@ -126,8 +126,8 @@ int trit_hip_layer_f16(int n, int k, const uint16_t *weights, const float *bias,
 /* y = x * W^T (+ bias, then max(y, 0) when relu): x is m x k f32, y m x n
  * f32, host memory. Replaces Dense::forward / forward_relu
  * (reference src/cpu/gemm.rs:500-542). Up to 8 rows run on the small-batch
- * GEMV kernels; more rows of a Q8_0, Q4_K or int8 layer with n % 128 == 0
- * run on the matrix cores (int8 MFMA), with the same bits. */
+ * GEMV kernels; more rows run on the matrix cores (int8 MFMA for the
+ * integer kinds, f32 MFMA for the float-math ones), with the same bits. */
 int trit_hip_layer_forward(const TritHipLayer *layer, const float *x, int m, int relu, float *y);
 
 /* The same on device pointers, enqueued on `stream` (a hipStream_t; NULL:
@@ -143,9 +143,10 @@ int trit_hip_layer_forward_device(const TritHipLayer *layer, const float *x, int
  * harnesses that forbid it). The activations of 2 or more rows are
  * quantized into one 4 MiB array per device that is part of the library
  * (its address found by trit_hip_init on that device, else by the first
- * call there), not into a per-thread buffer the library grows. A product
- * whose quantized rows need more than that fails with an error naming the
- * bytes it needs. All calls on one device share the array and it keeps the
+ * call there), not into a per-thread buffer the library grows. A Q8_0, Q4_K
+ * or int8 product whose quantized rows need more than that fails with an
+ * error naming the bytes it needs; ternary and float-math products of more
+ * rows than it holds run in passes. All calls on one device share the array and it keeps the
  * last call's contents: calls on one device must not overlap (queue them
  * on one stream). Results are trit_hip_layer_forward_device's, bit for
  * bit. Call trit_hip_init on the calling thread first (it creates the
