@@ -1696,11 +1696,12 @@ void ensure_rows(SessionImpl& S, int rows) {
     S.att_arrived.alloc((size_t)rows * c.kv_heads * 4);
     const int kmax = std::max(std::max(c.d, qd), c.ffn);
     size_t scratch = std::max(gemm_scratch_bytes(rows, kmax), gemv_scratch_bytes(8, kmax));
-    // Float-math linears of many rows: their operand copy.
+    // Of many rows: float-math linears' operand copy, ternary linears' padded codes.
     const DecoderImpl& D = *S.dec;
     for (int l = 0; l < c.layers && rows > 8; ++l)
         for (const Layer* L : {D.qkv[l].get(), D.o[l].get(), D.gate_up[l].get(), D.down[l].get()})
-            if (float_kind(L->kind)) scratch = std::max(scratch, gemm_float_scratch_want(rows, L->k));
+            scratch = std::max(scratch, float_kind(L->kind) ? gemm_float_scratch_want(rows, L->k)
+                                                            : gemm_scratch_bytes(*L, rows));
     S.gemm_scratch.alloc(scratch);
     TRIT_HIP(hipMemset(S.att_arrived.ptr, 0, (size_t)rows * c.kv_heads * 4));
     S.rows_cap = rows;

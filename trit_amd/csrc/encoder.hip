@@ -321,7 +321,7 @@ void encoder_product(const Layer& L, float* x, int m, float* y, const float* res
         conv = nullptr;
     }
     if (whole) {
-        const size_t need = gemm_scratch_bytes(m, L.k);
+        const size_t need = gemm_scratch_bytes(L, m);
         if (scratch.bytes < need) scratch.alloc(need);
         return gemm_int(L, a, scratch.ptr, s, conv);
     }

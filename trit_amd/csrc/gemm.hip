@@ -86,9 +86,19 @@ __global__ __launch_bounds__(WAVE) void row_norm_kernel(const float* __restrict_
     if (lane == 0) inv[row] = 1.0f / __builtin_sqrtf(sum / (float)k + eps);
 }
 
+// Byte of activation code (row, col) in the ternary product's operand order:
+// blocks of 32 rows by one 128-group, in a block the four MFMA steps of 64
+// lanes x 16 codes (step s, lane (row, half h): columns 64 h + 16 s ..), so a
+// wave's operand load is 1 KB in one piece.
+__device__ __forceinline__ size_t ternary_code(int row, int col, int k) {
+    const int g = col / 128, h = col / 64 % 2, s = col / 16 % 4;
+    return (((size_t)(row / 32) * (k / 128) + g) * 4 + s) * 1024 + (h * 32 + row % 32) * 16 + col % 16;
+}
+
 // Trit's activation quantizer (src/cpu/kernels.rs:661-737), G/4 threads per
-// group, four values a thread; rows [m, mpad) get zero scales.
-template <int G, bool HALF>
+// group, four values a thread; rows [m, mpad) get zero scales. TERN: codes in
+// the ternary product's order, else row-major.
+template <int G, bool HALF, bool TERN = false>
 __global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__ x, int m, int mpad, int k,
                                                        const float* __restrict__ norm_w,
                                                        const float* __restrict__ inv, int8_t* __restrict__ xq,
@@ -118,7 +128,7 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__
     const float q = 1.0f / scale;
     const int c0 = act_code(v.x * q), c1 = act_code(v.y * q);
     const int c2 = act_code(v.z * q), c3 = act_code(v.w * q);
-    if (real) *(uint32_t*)(xq + (size_t)row * k + col) = pack4(c0, c1, c2, c3);
+    if (real) *(uint32_t*)(xq + (TERN ? ternary_code(row, col, k) : (size_t)row * k + col)) = pack4(c0, c1, c2, c3);
     if (live && col % G == 0) xs[(size_t)(col / G) * mpad + row] = real ? (HALF ? f16_round(scale) : scale) : 0.0f;
 }
 
@@ -926,8 +936,11 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_wide_kernel(
 // Ternary products of many rows: 2-bit codes, f32 scales a 128-group, the
 // same contract (dot of the codes minus one and the activation codes). A wave
 // owns 32 x rows by TN 32-row weight tiles, four waves a block (2 x 2); no LDS
-// and no barriers, every operand straight from global memory, three groups in
-// flight. The order of K inside a group is free (an integer dot): MFMA step s
+// and no barriers, every operand straight from global memory, four groups in
+// flight: what bounds it is the address lines of the loads, so the codes of x
+// are quantized into operand order (ternary_code) and the weight scales load
+// four groups at once (from row-major codes, each load touching 32 rows, 375
+// rows through 4096 x 1024 and 1024 x 4096 took 48 us; 37 us so). The order of K inside a group is free (an integer dot): MFMA step s
 // of a group takes the codes 64 h + 16 s .. + 15 for the half h of the lanes,
 // so a lane's 16 bytes of 2-bit codes are its four steps' operands, each dword
 // unpacked by shifts, a mask and a byte permute that looks up code - 1. The
@@ -935,7 +948,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_wide_kernel(
 // of the two scale vectors in the dots' register layout (one product rounded
 // once, as the vector multiply rounds it), which leaves a conversion and a
 // multiply-add an output to the vector ALUs.
-constexpr int TERN_DEPTH = 3;
+constexpr int TERN_DEPTH = 4;
 
 template <int TN>
 __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_ternary_kernel(const int8_t* __restrict__ xq,
@@ -960,7 +973,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_ternary_kernel(const int
     const int lr = lane % 32, h = lane / 32;
     const int m0 = bm * BM + 32 * (w % 2), n0 = (bn * 2 + w / 2) * 32 * TN;
     if (m0 >= m || n0 >= n) return;
-    const int8_t* xp = xq + (size_t)min(m0 + lr, m - 1) * k + 64 * h;
+    const int8_t* xp = xq + (size_t)(m0 / 32) * groups * 4096 + lane * 16;  // (rows past m: not stored)
     const float* xsp = xs + m0 + lr;  // mpad covers the tile's rows
     const uint8_t* wp[TN];
 #pragma unroll
@@ -969,14 +982,27 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_ternary_kernel(const int
     const float* wsp = scales + (size_t)min(n0 + 32 * (TN == 2 ? h : 0) + lr, n - 1) * groups;
     v4i av[TERN_DEPTH][4];
     uint4 bv[TERN_DEPTH][TN];
-    float xv[TERN_DEPTH], wv[TERN_DEPTH];
+    float xv[TERN_DEPTH], wv[TERN_DEPTH], wnext[TERN_DEPTH];
     auto fetch = [&](int g, int d) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) av[d][s] = *(const v4i*)(xp + (size_t)g * 128 + 16 * s);
+        for (int s = 0; s < 4; ++s) av[d][s] = *(const v4i*)(xp + (size_t)g * 4096 + 1024 * s);
         xv[d] = xsp[(size_t)g * mpad];
 #pragma unroll
         for (int j = 0; j < TN; ++j) bv[d][j] = *(const uint4*)(wp[j] + (size_t)g * 32);
-        wv[d] = wsp[g];
+    };
+    // The scales of groups g .. g + 3 (past the last: the last's again, not used).
+    static_assert(TERN_DEPTH == 4, "four groups' scales a load");
+    auto fetch_scales = [&](int g) {
+        if (groups % 4 == 0) {
+            const float4 f = *(const float4*)(wsp + min(g, groups - 4));
+            wnext[0] = f.x;
+            wnext[1] = f.y;
+            wnext[2] = f.z;
+            wnext[3] = f.w;
+        } else {
+#pragma unroll
+            for (int d = 0; d < TERN_DEPTH; ++d) wnext[d] = wsp[min(g + d, groups - 1)];
+        }
     };
     const v16i magic = dot_base();
     float t[TN][16];
@@ -987,7 +1013,11 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_ternary_kernel(const int
 #pragma unroll
     for (int d = 0; d < TERN_DEPTH; ++d)
         if (d < groups) fetch(d, d);
+    fetch_scales(0);
     for (int g0 = 0; g0 < groups; g0 += TERN_DEPTH) {
+#pragma unroll
+        for (int d = 0; d < TERN_DEPTH; ++d) wv[d] = wnext[d];
+        fetch_scales(g0 + TERN_DEPTH);
 #pragma unroll
         for (int d = 0; d < TERN_DEPTH; ++d) {
             const int g = g0 + d;
@@ -1048,14 +1078,18 @@ struct Scratch {
     int mpad;
 };
 
-Scratch carve(void* base, int m, int k) {
-    const int mpad = round_up(m, BM);
+// Rows of x codes a product's scratch holds: whole 32-row operand blocks for a
+// ternary layer (64 with the scales' padding).
+int code_rows(const Layer& L, int m) { return L.kind == TERNARY ? round_up(m, BM) : m; }
+
+Scratch carve(void* base, const Layer& L, int m) {
+    const int mpad = round_up(m, BM), k = L.k;
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
     char* p = (char*)base;
     Scratch s;
     s.mpad = mpad;
     s.xq = (int8_t*)p;
-    p += al((size_t)m * k);
+    p += al((size_t)code_rows(L, m) * k);
     s.xs = (float*)p;
     p += al((size_t)(k / 32) * mpad * 4);
     s.inv = (float*)p;
@@ -1152,15 +1186,17 @@ size_t gemm_scratch_bytes(int m, int k) {
     return al((size_t)m * k) + al((size_t)(k / 32) * mpad * 4) + al(mpad * 4);
 }
 
+size_t gemm_scratch_bytes(const Layer& L, int m) { return gemm_scratch_bytes(code_rows(L, m), L.k); }
+
 bool gemm_conv_supported(const Layer& L, const ConvInput& in) {
-    return !float_kind(L.kind) && L.k == 9 * in.channels && in.channels % 4 == 0 &&
+    return !float_kind(L.kind) && L.kind != TERNARY && L.k == 9 * in.channels && in.channels % 4 == 0 &&
            (size_t)9 * conv_pitch(in.channels) * 4 <= 64 * 1024;
 }
 
 void gemm_int(const Layer& L, const GemvArgs& a, void* scratch, hipStream_t s, const ConvInput* conv) {
     if (!gemm_supported(L, a)) fail("gemm: layer " + std::to_string(L.n) + "x" + std::to_string(L.k) +
                                     " is not a shape the matrix-core product takes");
-    const Scratch sc = carve(scratch, a.m, L.k);
+    const Scratch sc = carve(scratch, L, a.m);
     const float* inv = a.norm_inv;
     if (a.norm_w && !inv) {
         hipLaunchKernelGGL(row_norm_kernel, dim3(a.m), dim3(WAVE), 0, s, a.x, L.k, a.eps, sc.inv, a.skip);
@@ -1180,7 +1216,10 @@ void gemm_int(const Layer& L, const GemvArgs& a, void* scratch, hipStream_t s, c
         else
             hipLaunchKernelGGL((quantize_conv_kernel<128, false>), dim3(blocks), dim3(256), lds, s, *conv, a.m,
                                sc.mpad, sc.xq, sc.xs, a.skip);
-    } else if (G == 32)
+    } else if (L.kind == TERNARY)
+        hipLaunchKernelGGL((quantize_kernel<128, false, true>), dim3(qblocks), dim3(256), 0, s, a.x, a.m, sc.mpad, L.k,
+                           a.norm_w, inv, sc.xq, sc.xs, a.skip);
+    else if (G == 32)
         hipLaunchKernelGGL((quantize_kernel<32, true>), dim3(qblocks), dim3(256), 0, s, a.x, a.m, sc.mpad, L.k,
                            a.norm_w, inv, sc.xq, sc.xs, a.skip);
     else

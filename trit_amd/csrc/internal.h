@@ -208,14 +208,16 @@ inline size_t gemm_float_scratch_want(int m, int k) {
     return all < cap ? all : least > cap ? least : cap;
 }
 void gemm_float_mfma(const Layer& L, GemvArgs a, void* scratch, size_t scratch_bytes, hipStream_t s);
-// Integer products of any row count on the matrix cores (Q8_0, Q4_K, INT8;
-// k a multiple of the weight group, any n; the SwiGLU pair needs n / 2 a
-// multiple of 64). `scratch` holds gemm_scratch_bytes(m, k) bytes of
+// Integer products of any row count on the matrix cores (every integer kind;
+// k a multiple of the weight group, any n; the SwiGLU pair not for ternary, n / 2 a
+// multiple of 64). `scratch` holds gemm_scratch_bytes(L, m) bytes of
 // device memory the product may overwrite.
 bool gemm_supported(const Layer& L, const GemvArgs& a);
 size_t gemm_scratch_bytes(int m, int k);
 // conv: the rows are the im2col columns of a kernel-3, stride-2, padding-1
 // convolution of maps [bin][time][channel] (k = 9 * channels), quantized
+// The same for one layer (a ternary layer's rows are padded to 64).
+size_t gemm_scratch_bytes(const Layer& L, int m);
 // straight from them; a.x is not read.
 struct ConvInput {
     const float* in;

@@ -359,12 +359,12 @@ void forward_rows(const Layer& L, GemvArgs a, int m, hipStream_t s, Scratch get,
                 a.x = x + (size_t)r0 * L.k;
                 a.y = y + (size_t)r0 * L.n;
                 a.m = m - r0 < rows ? m - r0 : rows;
-                gemm_int(L, a, get(gemm_scratch_bytes(a.m, L.k)), s);
+                gemm_int(L, a, get(gemm_scratch_bytes(L, a.m)), s);
             }
             return;
         }
     } else if (m >= GEMM_MIN_ROWS && gemm_supported(L, a))
-        return gemm_int(L, a, get(gemm_scratch_bytes(m, L.k)), s);
+        return gemm_int(L, a, get(gemm_scratch_bytes(L, m)), s);
     if (m > 8 && !a.ev_start && !a.ev_stop && gemm_float_supported(L, a)) return gemm_float(L, a, s);
     if (m > 8 && !a.ev_start && !a.ev_stop && gemm_float_mfma_supported(L, a) &&
         gemm_float_scratch_bytes(1, L.k) <= spare) {
