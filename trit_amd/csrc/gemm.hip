@@ -940,7 +940,8 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_wide_kernel(
 // flight: what bounds it is the address lines of the loads, so the codes of x
 // are quantized into operand order (ternary_code) and the weight scales load
 // four groups at once (from row-major codes, each load touching 32 rows, 375
-// rows through 4096 x 1024 and 1024 x 4096 took 48 us; 37 us so). The order of K inside a group is free (an integer dot): MFMA step s
+// rows through 4096 x 1024 and 1024 x 4096 took 48 us; 37 us so). The order of
+// K inside a group is free (an integer dot): MFMA step s
 // of a group takes the codes 64 h + 16 s .. + 15 for the half h of the lanes,
 // so a lane's 16 bytes of 2-bit codes are its four steps' operands, each dword
 // unpacked by shifts, a mask and a byte permute that looks up code - 1. The
