@@ -127,6 +127,11 @@ enum Epilogue {
 struct GemvArgs {
     const float* x = nullptr;  // m x k f32 (device)
     int m = 1;
+    // The exact GELU on the output, before the residual add (the products of
+    // many rows only: gemm_int without the pair, gemm_float, gemm_float_mfma).
+    // (Here, beside m, it leaves the kernels' arguments as large as without it:
+    // eight bytes more cost the 8-row ternary product 0.2 us of 10.8.)
+    int gelu = 0;
     // RMSNorm applied to each row of x before quantization: x * (inv * w).
     const float* norm_w = nullptr;    // k floats or null
     const float* norm_inv = nullptr;  // m floats (exact mode) or null: computed in the block
@@ -148,11 +153,6 @@ struct GemvArgs {
     // Set by the integer products: the quantized rows' image.
     const uint8_t* pre = nullptr;
 };
-    // The exact GELU on the output, before the residual add (the products of
-    // many rows only: gemm_int without the pair, gemm_float, gemm_float_mfma).
-    // (Here, beside m, it leaves the kernels' arguments as large as without it:
-    // eight bytes more cost the 8-row ternary product 0.2 us of 10.8.)
-    int gelu = 0;
 
 // Launches `kernel`, with the start/stop events of `a` when it has them.
 template <typename K, typename... Args>
@@ -216,10 +216,10 @@ void gemm_float_mfma(const Layer& L, GemvArgs a, void* scratch, size_t scratch_b
 // device memory the product may overwrite.
 bool gemm_supported(const Layer& L, const GemvArgs& a);
 size_t gemm_scratch_bytes(int m, int k);
-// conv: the rows are the im2col columns of a kernel-3, stride-2, padding-1
-// convolution of maps [bin][time][channel] (k = 9 * channels), quantized
 // The same for one layer (a ternary layer's rows are padded to 64).
 size_t gemm_scratch_bytes(const Layer& L, int m);
+// conv: the rows are the im2col columns of a kernel-3, stride-2, padding-1
+// convolution of maps [bin][time][channel] (k = 9 * channels), quantized
 // straight from them; a.x is not read.
 struct ConvInput {
     const float* in;
