@@ -245,6 +245,7 @@ int blocks_for(size_t n) { return (int)std::min<size_t>((n + 255) / 256, 4096); 
 struct Workspace {
     std::mutex mu;
     DeviceMemory bufs[16];
+    HostStage host;
     DeviceMemory& get(int i, size_t bytes) {
         if (bufs[i].bytes < bytes) bufs[i].alloc(bytes);
         return bufs[i];
@@ -499,8 +500,7 @@ int trit_hip_encoder_encode(const TritHipEncoder* encoder, const float* mel, flo
         }
         layer_norm(x.as<float>(), P, d, e.norm(c.layers, 0), e.norm(c.layers, 1), NORM_EPS, xn.as<float>(), s);
         TRIT_HIP(hipGetLastError());
-        TRIT_HIP(hipMemcpyAsync(out, xn.ptr, (size_t)P * d * 4, hipMemcpyDeviceToHost, s));
-        TRIT_HIP(hipStreamSynchronize(s));
+        ws.host.download(out, xn.ptr, (size_t)P * d * 4, s);
         return 0;
     });
 }
@@ -647,8 +647,7 @@ int trit_hip_asr_encoder_encode(const TritHipAsrEncoder* encoder, const float* m
         encoder_product(*e.proj1, xn.as<float>(), t, att.as<float>(), nullptr, true, scratch, s);
         encoder_product(*e.proj2, att.as<float>(), t, hid.as<float>(), nullptr, false, scratch, s);
         TRIT_HIP(hipGetLastError());
-        TRIT_HIP(hipMemcpyAsync(out, hid.ptr, (size_t)t * c.out * 4, hipMemcpyDeviceToHost, s));
-        TRIT_HIP(hipStreamSynchronize(s));
+        ws.host.download(out, hid.ptr, (size_t)t * c.out * 4, s);
         return t;
     });
 }

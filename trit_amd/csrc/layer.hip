@@ -224,6 +224,40 @@ void layer_forward(const Layer& L, const GemvArgs& a, hipStream_t s) {
     return gemv_int(L, a, s);
 }
 
+HostStage::~HostStage() {
+    for (hipEvent_t e : done)
+        if (e) (void)hipEventDestroy(e);
+    if (slots) (void)hipHostFree(slots);
+}
+
+void HostStage::prepare() {
+    if (!slots) TRIT_HIP(hipHostMalloc(&slots, SLOT * SLOTS, hipHostMallocDefault));
+    for (hipEvent_t& e : done)
+        if (!e) TRIT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+}
+
+void HostStage::download(void* host, const void* device, size_t bytes, hipStream_t s) {
+    if (bytes < 2 * SLOT) {
+        TRIT_HIP(hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, s));
+        TRIT_HIP(hipStreamSynchronize(s));
+        return;
+    }
+    prepare();
+    const size_t n = (bytes + SLOT - 1) / SLOT;
+    auto size = [&](size_t i) { return i + 1 < n ? SLOT : bytes - i * SLOT; };
+    for (size_t i = 0; i < n + SLOTS - 1; ++i) {
+        if (i < n) {
+            TRIT_HIP(hipMemcpyAsync(slot(i), (const char*)device + i * SLOT, size(i), hipMemcpyDeviceToHost, s));
+            TRIT_HIP(hipEventRecord(done[i % SLOTS], s));
+        }
+        if (i + 1 >= (size_t)SLOTS) {  // SLOTS - 1 copies behind
+            const size_t j = i + 1 - SLOTS;
+            TRIT_HIP(hipEventSynchronize(done[j % SLOTS]));
+            memcpy((char*)host + j * SLOT, slot(j), size(j));
+        }
+    }
+}
+
 // Per-thread staging buffers of the host-pointer forward, and the scratch
 // of the calling thread's many-row products. A thread holds one set from a
 // pool; when the thread ends, its set goes back to the pool (no HIP call)
