@@ -131,9 +131,15 @@ int trit_hip_layer_f16(int n, int k, const uint16_t *weights, const float *bias,
 int trit_hip_layer_forward(const TritHipLayer *layer, const float *x, int m, int relu, float *y);
 
 /* The same on device pointers, enqueued on `stream` (a hipStream_t; NULL:
- * the library's stream), without a wait. Products of 2 or more rows use a
- * scratch buffer of the calling thread: calls from one thread must not
- * overlap on different streams. */
+ * the library's stream), without a wait. Products of 2 or more rows use
+ * scratch memory of the calling thread: calls from one thread must not
+ * overlap on different streams. While `stream` is being captured, ternary
+ * and float-math (k > 128) products of more than 8 rows are launches of 8
+ * rows (same bits, many times slower: 375 rows through 4096x1024 and
+ * 1024x4096 ternary layers take 778 us so, 37 us otherwise); the
+ * no-allocation call below is the one to capture. A graph captured from
+ * this call holds the address of the scratch of an integer product of 2 or
+ * more rows, which a larger integer product of the same thread replaces. */
 int trit_hip_layer_forward_device(const TritHipLayer *layer, const float *x, int m, int relu, float *y,
                                   void *stream);
 
@@ -162,8 +168,9 @@ int trit_hip_layer_forward_device_noalloc(const TritHipLayer *layer, const float
  * their activations in a pass of their own first, and start_event then
  * stamps that pass's start, so the interval covers the whole call. A
  * matrix-core product stamps its GEMM kernel (the activation quantization
- * runs before it, unstamped). Fails for more than 8 rows of a layer the
- * matrix cores do not take. */
+ * runs before it, unstamped). More than 8 rows only of Q8_0, Q4_K and int8
+ * layers (k a multiple of the weight group); fails for more than 8 rows of
+ * a ternary or float-math one. */
 int trit_hip_layer_forward_timed(const TritHipLayer *layer, const float *x, int m, int relu, float *y,
                                  void *stream, void *start_event, void *stop_event);
 

@@ -267,7 +267,9 @@ void HostStage::download(void* host, const void* device, size_t bytes, hipStream
 // profiler wrapped around it) may already have shut down.
 struct Staging {
     int device = -1;
-    DeviceMemory x, y, scratch;
+    DeviceMemory x, y;
+    DeviceMemory scratch;  // the integer products' quantized rows; a captured graph may hold its address
+    DeviceMemory passes;   // the operands of products that run in passes (staging_passes); no graph holds it
 };
 
 struct StagingPool {
@@ -349,20 +351,26 @@ void* noalloc_scratch(int dev) {
     return g_scratch_ptr[dev];
 }
 
-// Grows the calling thread's scratch to `need` bytes.
-void* staging_scratch(size_t need) {
-    Staging& g = staging();
-    if (g.scratch.bytes < need) {
-        // Work already queued may still use the old scratch.
+void* grown(DeviceMemory& mem, size_t need) {
+    if (mem.bytes < need) {
+        // Work already queued may still use the old memory.
         TRIT_HIP(hipDeviceSynchronize());
-        g.scratch.alloc(need);
+        mem.alloc(need);
     }
-    return g.scratch.ptr;
+    return mem.ptr;
 }
 
-// The scratch bytes a product queued on `s` may ask of staging_scratch
-// beyond what it cannot do without: none while `s` is being captured (a
-// growth would allocate, and the graph would keep the old address).
+// The calling thread's scratch, grown to `need` bytes.
+void* staging_scratch(size_t need) { return grown(staging().scratch, need); }
+
+// The same for the operand copies of float-math rows and the codes of ternary
+// rows, up to 64 MiB: memory of their own, so that they never move the scratch
+// whose address a graph captured from an integer product holds.
+void* staging_passes(size_t need) { return grown(staging().passes, need); }
+
+// The bytes a product queued on `s` may ask of staging_passes: none while
+// `s` is being captured (a growth would allocate, and the graph would keep
+// the old address).
 size_t staging_spare(hipStream_t s) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &status) != hipSuccess) {
@@ -375,11 +383,12 @@ size_t staging_spare(hipStream_t s) {
 // One product of m rows: the matrix-core product for many rows, else the
 // small-batch kernels in calls of up to 8 rows (2..8 rows of an integer
 // layer with their activations quantized once, in the scratch). `get`
-// gives the scratch of `need` bytes (staging_scratch, or the no-allocation
-// array). Products that take any amount of scratch get `spare` bytes at
-// most; 0: they run in the calls of up to 8 rows.
-template <class Scratch>
-void forward_rows(const Layer& L, GemvArgs a, int m, hipStream_t s, Scratch get, size_t spare) {
+// gives the scratch of `need` bytes, `passes` that of the products that run
+// in passes of what it holds (staging_scratch and staging_passes, or both
+// the no-allocation array): `spare` bytes at most; 0: those products run in
+// the calls of up to 8 rows.
+template <class Scratch, class Passes>
+void forward_rows(const Layer& L, GemvArgs a, int m, hipStream_t s, Scratch get, Passes passes, size_t spare) {
     a.m = m;
     if (m >= GEMM_MIN_ROWS && L.kind == TERNARY) {
         // Passes of whole 64-row tiles where 64 MiB or `spare` does not hold all rows.
@@ -393,7 +402,7 @@ void forward_rows(const Layer& L, GemvArgs a, int m, hipStream_t s, Scratch get,
                 a.x = x + (size_t)r0 * L.k;
                 a.y = y + (size_t)r0 * L.n;
                 a.m = m - r0 < rows ? m - r0 : rows;
-                gemm_int(L, a, get(gemm_scratch_bytes(L, a.m)), s);
+                gemm_int(L, a, passes(gemm_scratch_bytes(L, a.m)), s);
             }
             return;
         }
@@ -403,7 +412,7 @@ void forward_rows(const Layer& L, GemvArgs a, int m, hipStream_t s, Scratch get,
     if (m > 8 && !a.ev_start && !a.ev_stop && gemm_float_mfma_supported(L, a) &&
         gemm_float_scratch_bytes(1, L.k) <= spare) {
         const size_t bytes = std::min(spare, gemm_float_scratch_want(m, L.k));
-        return gemm_float_mfma(L, a, get(bytes), bytes, s);
+        return gemm_float_mfma(L, a, passes(bytes), bytes, s);
     }
     if (m >= 2 && !float_kind(L.kind)) {
         a.scratch_bytes = gemv_scratch_bytes(m < 8 ? m : 8, L.k);
@@ -765,7 +774,7 @@ int trit_hip_layer_forward_device(const TritHipLayer* layer, const float* x, int
         a.relu = relu;
         if (m <= 0) fail("m must be positive");
         const hipStream_t st = s ? (hipStream_t)s : stream();
-        forward_rows(*layer->layer, a, m, st, staging_scratch, m > 8 ? staging_spare(st) : 0);
+        forward_rows(*layer->layer, a, m, st, staging_scratch, staging_passes, m > 8 ? staging_spare(st) : 0);
         return 0;
     });
 }
@@ -790,13 +799,14 @@ int trit_hip_layer_forward_device_noalloc(const TritHipLayer* layer, const float
         a.y = y;
         a.relu = relu;
         const Layer& L = *layer->layer;
-        forward_rows(L, a, m, s ? (hipStream_t)s : stream(), [&](size_t need) -> void* {
+        const auto array = [&](size_t need) -> void* {
             if (need > NOALLOC_SCRATCH_BYTES)
                 fail("no-allocation forward: " + std::to_string(m) + " rows of a " + std::to_string(L.n) + "x" +
                      std::to_string(L.k) + " layer need " + std::to_string(need) + " bytes of scratch, more than the " +
                      std::to_string(NOALLOC_SCRATCH_BYTES) + " it holds");
             return base;
-        }, NOALLOC_SCRATCH_BYTES);
+        };
+        forward_rows(L, a, m, s ? (hipStream_t)s : stream(), array, array, NOALLOC_SCRATCH_BYTES);
         return 0;
     });
 }
@@ -813,7 +823,7 @@ int trit_hip_layer_forward_timed(const TritHipLayer* layer, const float* x, int 
         a.ev_start = (hipEvent_t)start_event;
         a.ev_stop = (hipEvent_t)stop_event;
         const hipStream_t st = s ? (hipStream_t)s : stream();
-        forward_rows(*layer->layer, a, m, st, staging_scratch, 0);
+        forward_rows(*layer->layer, a, m, st, staging_scratch, staging_passes, 0);
         return 0;
     });
 }
