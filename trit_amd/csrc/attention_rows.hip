@@ -131,6 +131,8 @@ __global__ __launch_bounds__(64 * W, W == 4 && (HD == 64 || sizeof(KV) == 2) ? 3
     // sum, at most 1.2e-38: with f16 values (|v| <= 65504) such a term is
     // below 7.7e-34, under half a step of any |out| >= 2^-80, and the chains
     // stop at kmax (nearer 0 they go on, below); f32 values take every key.
+    // (Sums of less than 1: the row's maximum is infinite or all its scores
+    // are NaN, every key weighs the same, and sum and chains go on.)
     const int kmax = a.causal ? min(tk, pos + row0 + nr) : tk;
     const int kend = sizeof(KV) == 2 ? kmax : tk;
     const int ntiles = (kend + TILE - 1) / TILE;
@@ -252,7 +254,11 @@ __global__ __launch_bounds__(64 * W, W == 4 && (HD == 64 || sizeof(KV) == 2) ? 3
             if (w == 0) add_chunk(c);
         }
     }
-    if (t < TILE) inv_of[t] = 1.0f / sum;
+    if (t < TILE) {
+        if (sum < 1.0f)
+            for (int key = kmax; key < tk; ++key) sum = sum + exp_trit(-INFINITY);
+        inv_of[t] = 1.0f / sum;
+    }
     __syncthreads();
     const float inv = inv_of[lr];
 
@@ -354,7 +360,7 @@ __global__ __launch_bounds__(64 * W, W == 4 && (HD == 64 || sizeof(KV) == 2) ? 3
         for (int v = 0; v < VE; ++v) {
             const int e = VE * (TILE * w + 4 * q + r) + v;
             float acc = out[v][r];
-            if (kend < tk && !(__builtin_fabsf(acc) >= 0x1p-80f)) {
+            if (kend < tk && (inv > 1.0f || !(__builtin_fabsf(acc) >= 0x1p-80f))) {
                 const float pm = exp_trit(-INFINITY) * inv;
                 for (int key = kend; key < tk; ++key)
                     acc = __builtin_fmaf(pm, (float)((const KV*)(V + (uint32_t)key * pitch))[e], acc);

@@ -1413,7 +1413,8 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_rows_kernel(
     // there every row's weight is exp_trit(-inf) ~ 1.2e-38, which leaves a
     // sum of at least 1 (the maximum key's exp(0)) unchanged, so scores,
     // exponentials and the sums stop at kmax; the p.V chains too where that
-    // is exact (below).
+    // is exact (below). (A row whose maximum is infinite, or whose scores
+    // are all NaN, has that weight at every key: its sum and chains go on.)
     const int kmax = causal ? min(tk, st->pos + row0 + nr) : tk;
     float* qh = sm;
     float* probs = sm + R * MAX_HD;
@@ -1496,6 +1497,8 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_rows_kernel(
             for (int q = 0; q < 4; ++q) cur[q] = nxt[q];
         }
         for (; j < kmax; ++j) sum = sum + pr[j];
+        if (sum < 1.0f)
+            for (; j < tk; ++j) sum = sum + exp_trit(-INFINITY);
         inv[threadIdx.x] = 1.0f / sum;
     }
     __syncthreads();
@@ -1541,7 +1544,8 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_rows_kernel(
                 acc[k] = __builtin_fmaf(probs[r * pitch + j], v, acc[k]);
             }
         }
-        // Keys past kmax: weight pm = exp_trit(-inf) * (1/sum) <= 1.2e-38.
+        // Keys past kmax: weight pm = exp_trit(-inf) * (1/sum), <= 1.2e-38
+        // where the sum is at least 1 (else all keys weigh the same).
         // With f16 values (|v| <= 65504) each term is below 7.7e-34, under
         // half a step of any |acc| >= 2^-80, so it leaves acc as it is;
         // a chain nearer 0, or f32 values, takes the terms in order.
@@ -1550,7 +1554,7 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_rows_kernel(
             for (int k = 0; k < MR; ++k) {
                 const int r = group + k * G;
                 if (r >= nr) break;
-                if (sizeof(KV) == 2 && __builtin_fabsf(acc[k]) >= 0x1p-80f) continue;
+                if (sizeof(KV) == 2 && __builtin_fabsf(acc[k]) >= 0x1p-80f && inv[r] <= 1.0f) continue;
                 const float pm = exp_trit(-INFINITY) * inv[r];
                 for (int jj = kmax; jj < tk; ++jj) acc[k] = __builtin_fmaf(pm, kv_load(V + (size_t)jj * hd + e), acc[k]);
             }
