@@ -312,6 +312,14 @@ __global__ void qk_rope_kernel(float* __restrict__ qkv, int stride, int heads, i
 // all threads the rotary pairs.
 constexpr int RH = 32;
 
+// Whether it takes `items` heads of rows: where the chip holds a block a head
+// at once, those blocks' one serial sum is shorter than this kernel's passes
+// over 32 heads. Of 32 heads a row, a block a head against this kernel: 64 rows
+// of head_dim 128 4.2 us against 8.5, 384 rows 9.7 and 9.7, 512 rows 12.0 and
+// 10.0; of 64 320 rows 5.5 and 5.9, 448 rows 6.8 and 6.6; of 32 (blocks of 64
+// threads all the same) 192 rows 4.3 and 4.1, 256 rows 4.8 and 4.5.
+bool rope_by_rows(int items, int hd) { return items >= (hd < 64 ? 7000 : 13000); }
+
 template <typename KV>
 __global__ __launch_bounds__(256) void qk_rope_rows_kernel(float* __restrict__ qkv, int stride, int rows, int heads,
                                                            int kvh, int hd, int qk_norm,
@@ -1850,7 +1858,7 @@ void forward(SessionImpl& S, int rows, hipStream_t s) {
                 using KV = std::remove_pointer_t<decltype(kc)>;
                 const size_t lo = (size_t)l * c.kv_heads * S.max_pos * hd;
                 const int items = rows * (c.heads + 2 * c.kv_heads);
-                if (rows > 1)
+                if (rope_by_rows(items, hd))
                     hipLaunchKernelGGL(qk_rope_rows_kernel<KV>, dim3((items + RH - 1) / RH), dim3(256),
                                        (size_t)(RH * (hd + 4) + RH) * 4, s, S.qkv.as<float>(), stride, rows, c.heads,
                                        c.kv_heads, hd, c.qk_norm, D.q_norm(l), D.k_norm(l), c.eps,
