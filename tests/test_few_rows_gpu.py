@@ -1,0 +1,34 @@
+"""Products of 9 to 17 rows on both sides of the rules that choose between two
+launches of up to 8 rows and the matrix cores, against the oracle, bit for bit;
+rows that start at any 4-byte boundary among them."""
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests.device_memory import Device
+from tests.test_float_rows_gpu import bits_equal, layer_and_weights
+from trit_amd import hip, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind,n,k", [
+    ("f16", 512, 512), ("f16", 513, 512), ("f16", 1024, 4096), ("f16", 1025, 512), ("f16", 40, 8192), ("f16", 64, 1024),
+    ("f32", 512, 1024), ("f32", 513, 2048), ("f32", 64, 2112), ("q8", 1024, 512), ("q8", 1025, 1024), ("q8", 513, 2304)])
+def test_float_rows(gpu, kind, n, k):
+    print(f"case few rows {kind} n={n} k={k}", flush=True)
+    layer, w = layer_and_weights(kind, n, k)
+    x = synth.activations(71, 17, k)
+    want = O.matmul_f32(x, w)
+    D = Device()
+    try:
+        y, dx = D.empty(17 * n * 4), D.upload(x)
+        odd = D.upload(np.concatenate([x.reshape(-1)[:1], x.reshape(-1)]))
+        for rows in (9, 12, 13, 16, 17):
+            for at in (dx, odd.value + 4):
+                hip.check(hip.lib().trit_hip_layer_forward_device(layer.h, at, rows, 0, y, None))
+                assert bits_equal(D.download(y, (rows, n)), want[:rows]), (rows, at)
+    finally:
+        D.free()
+        layer.free()

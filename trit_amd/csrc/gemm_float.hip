@@ -293,8 +293,33 @@ void launch_kind(const Layer& L, const GemvArgs& a, const float4* xt, hipStream_
 
 }  // namespace
 
+namespace {
+
+// Whether 9 to 16 rows are shorter as two launches of up to 8 (gemv_float's
+// chunked kernel, which stages aligned rows of whole 16-byte weight steps): a
+// layer of few outputs fills those with one pass over its weights, while here
+// the operand copy, and for Q8 the widening in every row tile, come on top.
+// Rows 9 and 16, two launches against this file's kernels: f16 512x512 7.0 and
+// 7.6 us against 8.3 and 8.8, 512x8192 38 and 49 against 48 and 48, 1024x4096 25
+// and 33 against 27 and 27, 2048x4096 42 and 59 against 29 and 31; Q8 512x1024
+// 9.0 and 10.5 against 12.6 and 13.1, 2048x1024 13.3 and 18.7 against 12.5 and
+// 13.1; f32 256x2048 16.7 and 19.3 against 17.9 and 18.2. f16 rows of 1024 and
+// 2048 have a kernel of their own there that is slower (14.6 and 21.1 against
+// 11.8 and 12.3).
+bool few_rows_by_eights(const Layer& L, const GemvArgs& a) {
+    if (a.m > 16 || a.gelu || ((uintptr_t)a.x & 15) != 0) return false;
+    const bool most = a.m <= 12;
+    switch (L.kind) {
+        case F16: return L.k % 128 == 0 && L.k != 1024 && L.k != 2048 && L.k >= 512 && L.n <= (most ? 1024 : 512);
+        case F32: return L.k % 64 == 0 && L.k >= 1024 && L.k <= 2048 && L.n <= 512 && most;
+        default: return L.k % 256 == 0 && L.k >= 512 && L.n <= (most || L.k <= 2048 ? 1024 : 512);
+    }
+}
+
+}  // namespace
+
 bool gemm_float_mfma_supported(const Layer& L, const GemvArgs& a) {
-    return float_kind(L.kind) && a.m >= 1 && !a.norm_w && a.epilogue != EPI_SILU_PAIR;
+    return float_kind(L.kind) && a.m >= 9 && !a.norm_w && a.epilogue != EPI_SILU_PAIR && !few_rows_by_eights(L, a);
 }
 
 size_t gemm_float_scratch_bytes(int m, int k) {

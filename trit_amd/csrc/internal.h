@@ -222,8 +222,9 @@ void gemv_float(const Layer& L, const GemvArgs& a, hipStream_t s);
 // SwiGLU pair): the same bits row by row.
 bool gemm_float_supported(const Layer& L, const GemvArgs& a);
 void gemm_float(const Layer& L, const GemvArgs& a, hipStream_t s);
-// Float-math products of any row count and k on the f32 matrix cores (no
-// prologue, no SwiGLU pair): the same bits. `scratch` is device memory the
+// Float-math products of 9 or more rows and any k on the f32 matrix cores (no
+// prologue, no SwiGLU pair; not where two launches of up to 8 rows are
+// shorter): the same bits. `scratch` is device memory the
 // product may overwrite: gemm_float_scratch_bytes(m, k) take all rows in
 // one pass, less takes passes of as many rows as fit (at least 16, or it
 // fails). gemm_float_scratch_want: what to give it, the whole up to 64 MiB.
