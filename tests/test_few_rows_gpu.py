@@ -32,3 +32,24 @@ def test_float_rows(gpu, kind, n, k):
     finally:
         D.free()
         layer.free()
+
+
+@pytest.mark.parametrize("n,k", [(1024, 3584), (2048, 4096), (1024, 4096), (1028, 4096), (1024, 5120), (31, 5120),
+                                 (64, 6144), (64, 6784), (64, 6912)])
+def test_ternary_rows(gpu, n, k):
+    print(f"case few rows ternary n={n} k={k}", flush=True)
+    codes, scales = synth.ternary_matrix(synth.seed_for(72, n), n, k)
+    layer = hip.Dense.ternary(codes, scales)
+    x = synth.activations(73, 17, k)
+    want = O.Ternary(codes, scales)(x)
+    D = Device()
+    try:
+        y, dx = D.empty(17 * n * 4), D.upload(x)
+        for rows in (9, 10, 12, 13, 16, 17):
+            hip.check(hip.lib().trit_hip_layer_forward_device(layer.h, dx, rows, 0, y, None))
+            assert bits_equal(D.download(y, (rows, n)), want[:rows]), rows
+            hip.check(hip.lib().trit_hip_layer_forward_device_noalloc(layer.h, dx, rows, 0, y, None))
+            assert bits_equal(D.download(y, (rows, n)), want[:rows]), rows
+    finally:
+        D.free()
+        layer.free()

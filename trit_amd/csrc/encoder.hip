@@ -315,7 +315,7 @@ void encoder_product(const Layer& L, float* x, int m, float* y, const float* res
         a.residual = residual;
         a.epilogue = EPI_RESIDUAL;
     }
-    const bool whole = m > 8 && gemm_supported(L, a);
+    const bool whole = m > 8 && gemm_supported(L, a) && !ternary_by_eights(L, a);
     if (conv && !quantized_from_maps(L, m, *conv)) {
         hipLaunchKernelGGL(conv2d_columns_kernel, dim3(blocks_for((size_t)m * L.k)), dim3(256), 0, s, conv->in, maps,
                            conv->bins, conv->times, conv->channels, x);

@@ -1181,6 +1181,12 @@ bool gemm_supported(const Layer& L, const GemvArgs& a) {
     return a.m >= 1;
 }
 
+bool ternary_by_eights(const Layer& L, const GemvArgs& a) {
+    if (L.kind != TERNARY || a.gelu || a.m < 9 || a.m > 16 || L.n % 4 != 0 || L.k > 6784) return false;
+    if (a.m == 9) return L.k >= 3584 && L.n <= 2048;
+    return L.n <= 1024 && L.k >= (a.m == 10 ? 4096 : a.m <= 12 ? 5120 : 6144);
+}
+
 size_t gemm_scratch_bytes(int m, int k) {
     const size_t mpad = (size_t)round_up(m, BM);
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };

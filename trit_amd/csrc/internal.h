@@ -240,6 +240,14 @@ void gemm_float_mfma(const Layer& L, GemvArgs a, void* scratch, size_t scratch_b
 // multiple of 64). `scratch` holds gemm_scratch_bytes(L, m) bytes of
 // device memory the product may overwrite.
 bool gemm_supported(const Layer& L, const GemvArgs& a);
+// Whether 9 to 16 rows of a ternary layer are shorter as two launches of up
+// to 8: long rows and few outputs, where the matrix-core kernel is one wave's
+// serial chain over the groups. 9 and 16 rows, two launches against it:
+// 1024x4096 13.5 and 17.0 us against 16.1 and 16.3, 1024x6784 19.2 and 21.7
+// against 23.7 and 23.8, 2048x6144 18.4 and 23.6 against 21.6 and 21.8,
+// 1024x2048 14.5 and 21.4 against 10.9 and 11.1. (8 rows of 6784 inputs are
+// near what that kernel's shared memory holds.)
+bool ternary_by_eights(const Layer& L, const GemvArgs& a);
 size_t gemm_scratch_bytes(int m, int k);
 // The same for one layer (a ternary layer's rows are padded to 64).
 size_t gemm_scratch_bytes(const Layer& L, int m);

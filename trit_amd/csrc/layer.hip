@@ -393,7 +393,7 @@ void forward_rows(const Layer& L, GemvArgs a, int m, hipStream_t s, Scratch get,
     if (m >= GEMM_MIN_ROWS && L.kind == TERNARY) {
         // Passes of whole 64-row tiles where 64 MiB or `spare` does not hold all rows.
         const size_t tile = gemm_scratch_bytes(64, L.k);
-        if (!a.ev_start && !a.ev_stop && gemm_supported(L, a) && tile <= spare) {
+        if (!a.ev_start && !a.ev_stop && gemm_supported(L, a) && !ternary_by_eights(L, a) && tile <= spare) {
             const size_t tiles = std::max<size_t>(1, std::min(spare, (size_t)64 << 20) / tile), all = (size_t)(m + 63) / 64;
             const int rows = (int)std::min((size_t)m, 64 * std::min(tiles, all));
             const float* x = a.x;
