@@ -1381,13 +1381,28 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_steps_one_kernel(const 
                              out + (size_t)b * d + (size_t)h * hd);
 }
 
+// Whether attention_steps_kernel is the shorter one for `blocks` blocks of at
+// most `most` keys: for few keys attention_one's value stages (32 KB of LDS,
+// two barriers each) are longer than what they hide. The lines lie where both
+// took the same; us, that kernel and attention_one (heads x head_dim x
+// sequences): 20x64x5 16 keys 5.1, 4.2 and 20x64x32 (past 512 blocks) 16 keys
+// 5.5, 6.9, 96 keys 14.4, 12.0; 8x32 24 keys 4.6, 4.9, 48 keys 5.6, 5.3; 8x128
+// 16 keys 6.4, 6.7, 64 keys 8.7, 8.6, 448 keys 26.8, 23.8; 4x192 96 keys 11.3,
+// 11.9, 320 keys 25.1, 25.1; 4x256 448 keys 32.6, 34.4, 4000 keys 472, 295.
+bool steps_short(int hd, int blocks, int most) {
+    if (hd == 64) return blocks > 512 && most <= 64;
+    if (hd < 64) return most <= (blocks > 512 ? 64 : 40);
+    if (hd < 192) return most <= (blocks > 512 ? 32 : 48);
+    return most <= (blocks > 256 ? 48 : 96) || (hd > 192 && (int64_t)blocks * most <= 9000);
+}
+
 // Sequences of at most `most` keys: on attention_one where its shared memory
-// holds them (about 7800 keys), else on attention_steps_kernel.
+// holds them (7928 keys) and it is the shorter, else on attention_steps_kernel.
 void launch_steps(const float* q, int qs, const StepsTable& table, int sequences, int d, int heads, int kvh, int hd,
                   int most, float* out, hipStream_t s) {
     const dim3 grid(heads, sequences);
     const size_t lds = attention_one_lds(most);
-    if (lds > 64 * 1024)
+    if (lds > 64 * 1024 || steps_short(hd, heads * sequences, most))
         hipLaunchKernelGGL(attention_steps_kernel, grid, dim3(ATT_THREADS), (size_t)(MAX_HD + most + ATT_THREADS) * 4, s, q,
                            qs, table, heads, kvh, hd, d, out);
     else if (hd == 64)
