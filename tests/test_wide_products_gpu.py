@@ -24,3 +24,11 @@ def test_wide(gpu, n, k, m):
     want = np.maximum(O.Int8(codes, sbits.view(np.float16).astype(np.float32), 32, True)(x) + bias, 0)
     assert np.array_equal(got.view(np.uint32), want.astype(np.float32).view(np.uint32))
     layer.free()
+
+
+# As above, where the 128 x 128 blocks start: more than 256 of them, or 160 with
+# long rows; and the last sizes before it.
+@pytest.mark.parametrize("n,k,m", [(33024, 32, 9), (32768, 32, 9), (2656, 64, 1601), (96, 160, 32900), (2656, 416, 1665),
+                                   (480, 2080, 5100), (480, 2016, 5100), (20480, 3104, 64), (20480, 3040, 17)])
+def test_both_sides_of_the_rule(gpu, n, k, m):
+    test_wide(gpu, n, k, m)

@@ -1109,11 +1109,19 @@ bool narrow(int n, int mb) {
 }
 
 // Whether a plain product takes gemm_wide_kernel: k not a multiple of 128, and
-// 128 x 128 blocks for most CUs (n 480, k 4320, with the GELU: 24000 rows, 752
-// blocks, 218 us against 337 us for gemm_kernel; 6000 rows, 196 blocks, 95 us
-// against 111). For other k the 64 x 64 blocks are faster (1564 x 6144 x 2048,
-// 624 blocks: 68 us against 82).
-bool wide(int nb, int m, int k) { return k % KD != 0 && (int64_t)nb * ((m + 127) / 128) >= 160; }
+// more 128 x 128 blocks than gemm_kernel's, two a CU, hold at once (256: past
+// them that kernel starts a second round), or rows long enough that half the
+// loads a byte pay earlier. gemm_kernel against it, us (quantizer included): n
+// 480, 384 blocks, k 32 15.8, 13.1, k 1056 61.7, 48.9, k 4320 244, 157; 192
+// blocks, k 160 13.2, 14.7, k 1056 35.4, 35.3, k 2080 58.3, 57.1, k 4320 119,
+// 105; one block row of at most 64 rows (half of each block unused), n 20480, 160
+// blocks, k 1056 23.2, 26.8, k 2080 38.4, 42.9, k 3104 64.3, 58.3. For k a
+// multiple of 128 the 64 x 64 blocks are faster (1564 x 6144 x 2048, 624 blocks:
+// 68 us against 82).
+bool wide(int nb, int m, int k) {
+    const int64_t blocks = (int64_t)nb * ((m + 127) / 128);
+    return k % KD != 0 && (blocks > 256 || (blocks >= 160 && k >= (m > 64 ? 2048 : 3072)));
+}
 
 template <int G, bool HALF, int P>
 void launch_gemm(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStream_t s) {
