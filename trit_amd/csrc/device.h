@@ -74,6 +74,25 @@ __device__ __forceinline__ float gelu_trit(float v) {
     return (0.5f * v) * (v >= 0.0f ? 2.0f - tail : tail);
 }
 
+// N outputs of one row of a many-row product, of the columns `col`, before
+// their store: bias, relu, the GELU. (GELU a constant: its code in the kernels
+// of products without one, branched over, cost them 0.2-0.5 us of 8-12.)
+template <bool GELU, int N>
+__device__ __forceinline__ void finish_outputs(float (&v)[N], const float* bias, const int (&col)[N], int relu) {
+    if (bias) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = v[i] + bias[col[i]];
+    }
+    if (relu) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = __builtin_fmaxf(v[i], 0.0f);
+    }
+    if (GELU) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = gelu_trit(v[i]);
+    }
+}
+
 // Activation code: round to nearest even, then the +-127 limits; a NaN
 // becomes -127 as cvtps2dq + clamp gives it (src/cpu/v2/quantize.rs:140-149).
 __device__ __forceinline__ int act_code(float scaled) {

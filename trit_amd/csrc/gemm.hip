@@ -257,7 +257,7 @@ __device__ __forceinline__ void read_scales(const float* xs, const float* ws, in
     s.w1 = ws[c1];
 }
 
-template <int G, bool HALF, int P, bool TAIL>
+template <int G, bool HALF, int P, bool TAIL, bool GELU>
 __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(const int8_t* __restrict__ xq,
                                                                const float* __restrict__ xs, int m, int mpad,
                                                                const int8_t* __restrict__ codes,
@@ -455,26 +455,15 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(const int8_t* __r
     for (int r = 0; r < 16; ++r) {
         const int row = m0 + 8 * (r / 4) + 4 * h + r % 4;
         if (row >= m) continue;
-        float v0 = t0[r], v1 = t1[r];
-        if (bias) {
-            v0 = v0 + bias[min(r0 + lr, n - 1)];  // columns past n are not stored
-            v1 = v1 + bias[min(r1 + lr, n - 1)];
-        }
-        if (a.relu) {
-            v0 = __builtin_fmaxf(v0, 0.0f);
-            v1 = __builtin_fmaxf(v1, 0.0f);
-        }
-        if (P == 1 && a.gelu) {
-            v0 = gelu_trit(v0);
-            v1 = gelu_trit(v1);
-        }
+        float v[2] = {t0[r], t1[r]};
+        finish_outputs<GELU>(v, bias, {min(r0 + lr, n - 1), min(r1 + lr, n - 1)}, a.relu);  // columns past n are not stored
         if (P == 2) {
-            a.y[(size_t)row * ldy + r0 + lr] = silu_trit(v0) * v1;
+            a.y[(size_t)row * ldy + r0 + lr] = silu_trit(v[0]) * v[1];
             continue;
         }
         const size_t i0 = (size_t)row * ldy + r0 + lr, i1 = (size_t)row * ldy + r1 + lr;
-        if (r0 + lr < n) a.y[i0] = a.epilogue == EPI_RESIDUAL ? a.residual[i0] + v0 : v0;
-        if (r1 + lr < n) a.y[i1] = a.epilogue == EPI_RESIDUAL ? a.residual[i1] + v1 : v1;
+        if (r0 + lr < n) a.y[i0] = a.epilogue == EPI_RESIDUAL ? a.residual[i0] + v[0] : v[0];
+        if (r1 + lr < n) a.y[i1] = a.epilogue == EPI_RESIDUAL ? a.residual[i1] + v[1] : v[1];
     }
 }
 
@@ -521,7 +510,7 @@ __device__ __forceinline__ void load4_to_lds(const void* g, void* l) {
     asm volatile("global_load_lds_dword %0, off" ::"v"(g), "{m0}"(lds_address(l)) : "memory");
 }
 
-template <int G, bool HALF, int P, int TW>
+template <int G, bool HALF, int P, int TW, bool GELU>
 __global__ __launch_bounds__(GEMM_THREADS, TW == 2 ? 3 : 4) void gemm_dma_kernel(
     const int8_t* __restrict__ xq, const float* __restrict__ xs, int m, int mpad, const int8_t* __restrict__ codes,
     const void* __restrict__ scales, const float* __restrict__ bias, int n, int k, int nb, int mb, GemvArgs a) {
@@ -729,26 +718,23 @@ __global__ __launch_bounds__(GEMM_THREADS, TW == 2 ? 3 : 4) void gemm_dma_kernel
     for (int r = 0; r < 16; ++r) {
         const int row = m0 + 8 * (r / 4) + 4 * h + r % 4;
         if (row >= m) continue;
-        float v0 = t0[r], v1 = t1[r];
-        if (bias) {
-            v0 = v0 + bias[min(r0 + lr, n - 1)];
-            v1 = v1 + bias[min(r1 + lr, n - 1)];
+        float v[TW] = {t0[r]};
+        int col[TW] = {min(r0 + lr, n - 1)};
+        if constexpr (TW == 2) {
+            v[1] = t1[r];
+            col[1] = min(r1 + lr, n - 1);
         }
-        if (a.relu) {
-            v0 = __builtin_fmaxf(v0, 0.0f);
-            v1 = __builtin_fmaxf(v1, 0.0f);
-        }
-        if (P == 1 && a.gelu) {
-            v0 = gelu_trit(v0);
-            v1 = gelu_trit(v1);
-        }
-        if (P == 2) {
-            a.y[(size_t)row * ldy + r0 + lr] = silu_trit(v0) * v1;
+        finish_outputs<GELU>(v, bias, col, a.relu);
+        if constexpr (P == 2) {
+            a.y[(size_t)row * ldy + r0 + lr] = silu_trit(v[0]) * v[1];
             continue;
         }
-        const size_t i0 = (size_t)row * ldy + r0 + lr, i1 = (size_t)row * ldy + r1 + lr;
-        if (r0 + lr < n) a.y[i0] = a.epilogue == EPI_RESIDUAL ? a.residual[i0] + v0 : v0;
-        if (TW == 2 && r1 + lr < n) a.y[i1] = a.epilogue == EPI_RESIDUAL ? a.residual[i1] + v1 : v1;
+        const size_t i0 = (size_t)row * ldy + r0 + lr;
+        if (r0 + lr < n) a.y[i0] = a.epilogue == EPI_RESIDUAL ? a.residual[i0] + v[0] : v[0];
+        if constexpr (TW == 2) {
+            const size_t i1 = (size_t)row * ldy + r1 + lr;
+            if (r1 + lr < n) a.y[i1] = a.epilogue == EPI_RESIDUAL ? a.residual[i1] + v[1] : v[1];
+        }
     }
 }
 
@@ -767,6 +753,7 @@ struct alignas(16) WStage {
     alignas(16) uint32_t ws[3 * 128];
 };
 
+template <bool GELU>
 __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_wide_kernel(
     const int8_t* __restrict__ xq, const float* __restrict__ xs, int m, int mpad, const int8_t* __restrict__ codes,
     const void* __restrict__ scales, const float* __restrict__ bias, int n, int k, int nb, int mb, GemvArgs a) {
@@ -914,22 +901,11 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_wide_kernel(
         for (int r = 0; r < 16; ++r) {
             const int row = mbase + (w % 2) * 64 + 32 * i + 8 * (r / 4) + 4 * h + r % 4;
             if (row >= m) continue;
-            float v0 = acc[i][0][r], v1 = acc[i][1][r];
-            if (bias) {
-                v0 = v0 + bias[min(r0 + lr, n - 1)];
-                v1 = v1 + bias[min(r1 + lr, n - 1)];
-            }
-            if (a.relu) {
-                v0 = __builtin_fmaxf(v0, 0.0f);
-                v1 = __builtin_fmaxf(v1, 0.0f);
-            }
-            if (a.gelu) {
-                v0 = gelu_trit(v0);
-                v1 = gelu_trit(v1);
-            }
+            float v[2] = {acc[i][0][r], acc[i][1][r]};
+            finish_outputs<GELU>(v, bias, {min(r0 + lr, n - 1), min(r1 + lr, n - 1)}, a.relu);
             const size_t i0 = (size_t)row * n + r0 + lr, i1 = (size_t)row * n + r1 + lr;
-            if (r0 + lr < n) a.y[i0] = a.epilogue == EPI_RESIDUAL ? a.residual[i0] + v0 : v0;
-            if (r1 + lr < n) a.y[i1] = a.epilogue == EPI_RESIDUAL ? a.residual[i1] + v1 : v1;
+            if (r0 + lr < n) a.y[i0] = a.epilogue == EPI_RESIDUAL ? a.residual[i0] + v[0] : v[0];
+            if (r1 + lr < n) a.y[i1] = a.epilogue == EPI_RESIDUAL ? a.residual[i1] + v[1] : v[1];
         }
 }
 
@@ -951,7 +927,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_wide_kernel(
 // multiply-add an output to the vector ALUs.
 constexpr int TERN_DEPTH = 4;
 
-template <int TN>
+template <int TN, bool GELU>
 __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_ternary_kernel(const int8_t* __restrict__ xq,
                                                                        const float* __restrict__ xs, int m, int mpad,
                                                                        const uint8_t* __restrict__ codes,
@@ -1060,12 +1036,10 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_ternary_kernel(const int
         for (int r = 0; r < 16; ++r) {
             const int row = m0 + 8 * (r / 4) + 4 * h + r % 4;
             if (row >= m) continue;
-            float v = t[j][r];
-            if (bias) v = v + bias[col];
-            if (a.relu) v = __builtin_fmaxf(v, 0.0f);
-            if (a.gelu) v = gelu_trit(v);
+            float v[1] = {t[j][r]};
+            finish_outputs<GELU>(v, bias, {col}, a.relu);
             const size_t at = (size_t)row * n + col;
-            a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v : v;
+            a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v[0] : v[0];
         }
     }
 }
@@ -1123,14 +1097,14 @@ bool wide(int nb, int m, int k) {
     return k % KD != 0 && (blocks > 256 || (blocks >= 160 && k >= (m > 64 ? 2048 : 3072)));
 }
 
-template <int G, bool HALF, int P>
+template <int G, bool HALF, int P, bool GELU>
 void launch_gemm(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStream_t s) {
     const int nb = P == 1 ? (L.n + 127) / 128 : (L.n / 2) / 64;
     const int mb = sc.mpad / BM;
     if constexpr (G == 32 && P == 1) {
         if (wide(nb, a.m, L.k)) {
             const int mb2 = (a.m + 127) / 128;
-            launch_timed(a, gemm_wide_kernel, dim3(nb * mb2), dim3(GEMM_THREADS), 0, s, (const int8_t*)sc.xq,
+            launch_timed(a, gemm_wide_kernel<GELU>, dim3(nb * mb2), dim3(GEMM_THREADS), 0, s, (const int8_t*)sc.xq,
                          (const float*)sc.xs, a.m, sc.mpad, L.codes.as<int8_t>(), (const void*)L.scales.ptr,
                          L.bias.as<float>(), L.n, L.k, nb, mb2, a);
             TRIT_HIP(hipGetLastError());
@@ -1140,7 +1114,7 @@ void launch_gemm(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStream
     if constexpr (P == 1) {
         if (L.k % KD == 0 && narrow(L.n, mb)) {
             const int nb1 = (L.n + 63) / 64;
-            launch_timed(a, gemm_dma_kernel<G, HALF, P, 1>, dim3(nb1 * mb), dim3(GEMM_THREADS), 0, s,
+            launch_timed(a, gemm_dma_kernel<G, HALF, P, 1, GELU>, dim3(nb1 * mb), dim3(GEMM_THREADS), 0, s,
                          (const int8_t*)sc.xq, (const float*)sc.xs, a.m, sc.mpad, L.codes.as<int8_t>(),
                          (const void*)L.scales.ptr, L.bias.as<float>(), L.n, L.k, nb1, mb, a);
             TRIT_HIP(hipGetLastError());
@@ -1148,11 +1122,11 @@ void launch_gemm(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStream
         }
     }
     if (L.k % KD == 0)
-        launch_timed(a, gemm_dma_kernel<G, HALF, P, 2>, dim3(nb * mb), dim3(GEMM_THREADS), 0, s,
+        launch_timed(a, gemm_dma_kernel<G, HALF, P, 2, GELU>, dim3(nb * mb), dim3(GEMM_THREADS), 0, s,
                      (const int8_t*)sc.xq, (const float*)sc.xs, a.m, sc.mpad, L.codes.as<int8_t>(),
                      (const void*)L.scales.ptr, L.bias.as<float>(), L.n, L.k, nb, mb, a);
     else if constexpr (G == 32)
-        launch_timed(a, gemm_kernel<G, HALF, P, true>, dim3(nb * mb), dim3(GEMM_THREADS), 0, s,
+        launch_timed(a, gemm_kernel<G, HALF, P, true, GELU>, dim3(nb * mb), dim3(GEMM_THREADS), 0, s,
                      (const int8_t*)sc.xq, (const float*)sc.xs, a.m, sc.mpad, L.codes.as<int8_t>(),
                      (const void*)L.scales.ptr, L.bias.as<float>(), L.n, L.k, nb, mb, a);
     TRIT_HIP(hipGetLastError());
@@ -1165,9 +1139,9 @@ void launch_ternary(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStr
     auto go = [&](auto TN_) {
         constexpr int TN = decltype(TN_)::value;
         const int nb = (L.n + 64 * TN - 1) / (64 * TN);
-        launch_timed(a, gemm_ternary_kernel<TN>, dim3(nb * mb), dim3(GEMM_THREADS), 0, s, (const int8_t*)sc.xq,
-                     (const float*)sc.xs, a.m, sc.mpad, L.codes.as<uint8_t>(), L.scales.as<float>(),
-                     L.bias.as<float>(), L.n, L.k, nb, mb, a);
+        launch_timed(a, a.gelu ? gemm_ternary_kernel<TN, true> : gemm_ternary_kernel<TN, false>, dim3(nb * mb),
+                     dim3(GEMM_THREADS), 0, s, (const int8_t*)sc.xq, (const float*)sc.xs, a.m, sc.mpad,
+                     L.codes.as<uint8_t>(), L.scales.as<float>(), L.bias.as<float>(), L.n, L.k, nb, mb, a);
     };
     if ((int64_t)((L.n + 127) / 128) * mb >= 256) go(std::integral_constant<int, 2>{});
     else go(std::integral_constant<int, 1>{});
@@ -1242,13 +1216,11 @@ void gemm_int(const Layer& L, const GemvArgs& a, void* scratch, hipStream_t s, c
                            a.norm_w, inv, sc.xq, sc.xs, a.skip);
     TRIT_HIP(hipGetLastError());
     if (L.kind == TERNARY) return launch_ternary(L, a, sc, s);
-    const bool pair = a.epilogue == EPI_SILU_PAIR;
-    if (G == 32) {
-        if (pair) return launch_gemm<32, true, 2>(L, a, sc, s);
-        return launch_gemm<32, true, 1>(L, a, sc, s);
-    }
-    if (pair) return launch_gemm<128, false, 2>(L, a, sc, s);
-    return launch_gemm<128, false, 1>(L, a, sc, s);
+    if (a.epilogue == EPI_SILU_PAIR)
+        return G == 32 ? launch_gemm<32, true, 2, false>(L, a, sc, s) : launch_gemm<128, false, 2, false>(L, a, sc, s);
+    if (a.gelu)
+        return G == 32 ? launch_gemm<32, true, 1, true>(L, a, sc, s) : launch_gemm<128, false, 1, true>(L, a, sc, s);
+    return G == 32 ? launch_gemm<32, true, 1, false>(L, a, sc, s) : launch_gemm<128, false, 1, false>(L, a, sc, s);
 }
 
 }  // namespace trit

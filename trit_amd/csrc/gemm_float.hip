@@ -157,7 +157,7 @@ __device__ __forceinline__ void widen(const Raw<K>& r, float (&f)[4]) {
 }
 
 // Output tile: TM x TN tiles of 16 x 16 a block.
-template <int K, bool VEC, int TM, int TN>
+template <int K, bool VEC, int TM, int TN, bool GELU>
 __global__ __launch_bounds__(THREADS, 2) void float_mfma_kernel(const float4* __restrict__ xt, int tiles, int nb,
                                                                 const typename WT<K>::E* __restrict__ w,
                                                                 const float* __restrict__ scales,
@@ -259,12 +259,10 @@ __global__ __launch_bounds__(THREADS, 2) void float_mfma_kernel(const float4* __
     for (int e = threadIdx.x; e < BM * BN; e += THREADS) {
         const int row = bm * BM + e / BN, col = bn * BN + e % BN;
         if (row >= a.m || col >= n) continue;
-        float v = (part[0][e] + part[2][e]) + (part[1][e] + part[3][e]);
-        if (bias) v = v + bias[col];
-        if (a.relu) v = __builtin_fmaxf(v, 0.0f);
-        if (a.gelu) v = gelu_trit(v);
+        float v[1] = {(part[0][e] + part[2][e]) + (part[1][e] + part[3][e])};
+        finish_outputs<GELU>(v, bias, {col}, a.relu);
         const size_t at = (size_t)row * n + col;
-        a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v : v;
+        a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v[0] : v[0];
     }
 }
 
@@ -277,9 +275,9 @@ void launch_tiles(const Layer& L, const GemvArgs& a, const float4* xt, hipStream
     auto go = [&](auto TN_) {
         constexpr int TN = decltype(TN_)::value;
         const int nbn = (L.n + TN * TILE - 1) / (TN * TILE);
-        hipLaunchKernelGGL((float_mfma_kernel<K, VEC, 2, TN>), dim3(nbn * nbm), dim3(THREADS), 0, s, xt, tiles, nb,
-                           L.codes.as<E>(), K == WK_Q8 ? L.scales.as<float>() : nullptr, L.bias.as<float>(), L.n,
-                           L.k, nbn, nbm, a);
+        hipLaunchKernelGGL((a.gelu ? float_mfma_kernel<K, VEC, 2, TN, true> : float_mfma_kernel<K, VEC, 2, TN, false>),
+                           dim3(nbn * nbm), dim3(THREADS), 0, s, xt, tiles, nb, L.codes.as<E>(),
+                           K == WK_Q8 ? L.scales.as<float>() : nullptr, L.bias.as<float>(), L.n, L.k, nbn, nbm, a);
     };
     if ((int64_t)((L.n + 63) / 64) * nbm >= 256) go(std::integral_constant<int, 4>{});
     else go(std::integral_constant<int, 1>{});

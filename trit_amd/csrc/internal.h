@@ -152,9 +152,8 @@ struct GemvArgs {
     const float* x = nullptr;  // m x k f32 (device)
     int m = 1;
     // The exact GELU on the output, before the residual add (the products of
-    // many rows only: gemm_int without the pair, gemm_float, gemm_float_mfma).
-    // (Here, beside m, it leaves the kernels' arguments as large as without it:
-    // eight bytes more cost the 8-row ternary product 0.2 us of 10.8.)
+    // many rows only: gemm_int without the pair, gemm_float, gemm_float_mfma,
+    // whose launches pick the kernel compiled with it).
     int gelu = 0;
     // RMSNorm applied to each row of x before quantization: x * (inv * w).
     const float* norm_w = nullptr;    // k floats or null
