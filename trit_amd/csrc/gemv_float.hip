@@ -299,7 +299,7 @@ __global__ __launch_bounds__(THREADS) void float_chunked_kernel(const typename W
 // rows; a thread holds its column's 16 lane chains (S steps each) in
 // registers and runs them over the rows, then the tree16 order of the
 // small-batch kernels, so every row gets their bits.
-template <int K, int S>
+template <int K, int S, bool GELU>
 __global__ __launch_bounds__(THREADS) void float_rows_kernel(const typename WT<K>::E* __restrict__ w,
                                                              const float* __restrict__ scales,
                                                              const float* __restrict__ bias, int n, int k, GemvArgs a) {
@@ -332,15 +332,13 @@ __global__ __launch_bounds__(THREADS) void float_rows_kernel(const typename WT<K
         float h[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) h[i] = l[i] + l[i + 8];
-        float v = ((h[0] + h[4]) + (h[2] + h[6])) + ((h[1] + h[5]) + (h[3] + h[7]));
-        if (a.gelu) {
-            if (bias) v = v + bias[col];
-            if (a.relu) v = __builtin_fmaxf(v, 0.0f);
+        float v[1] = {((h[0] + h[4]) + (h[2] + h[6])) + ((h[1] + h[5]) + (h[3] + h[7]))};
+        if constexpr (GELU) {
+            finish_outputs<true>(v, bias, {col}, a.relu);
             const size_t at = (size_t)f * n + col;
-            v = gelu_trit(v);
-            a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v : v;
+            a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v[0] : v[0];
         } else {
-            store_out(a, bias, n, f, col, v);
+            store_out(a, bias, n, f, col, v[0]);
         }
     }
 }
@@ -442,8 +440,8 @@ void gemm_float(const Layer& L, const GemvArgs& a, hipStream_t s) {
         constexpr int K = decltype(K_)::value, S = decltype(S_)::value;
         using E = typename WT<K>::E;
         const dim3 grid((L.n + THREADS - 1) / THREADS, (a.m + 63) / 64);
-        launch_timed(a, float_rows_kernel<K, S>, grid, dim3(THREADS), 0, s, L.codes.as<E>(),
-                     K == WK_Q8 ? L.scales.as<float>() : nullptr, L.bias.as<float>(), L.n, L.k, a);
+        launch_timed(a, a.gelu ? float_rows_kernel<K, S, true> : float_rows_kernel<K, S, false>, grid, dim3(THREADS), 0,
+                     s, L.codes.as<E>(), K == WK_Q8 ? L.scales.as<float>() : nullptr, L.bias.as<float>(), L.n, L.k, a);
     };
     auto by_steps = [&](auto K_) {
         const int steps = chain_steps(L.k);
