@@ -299,13 +299,34 @@ bool quantized_from_maps(const Layer& L, int m, const ConvInput& conv) {
     return m > 8 && gemm_supported(L, a) && gemm_conv_supported(L, conv);
 }
 
+// The scratch encoder_product needs for m rows of a layer.
+size_t product_scratch(const Layer& L, int m) {
+    GemvArgs a;
+    a.m = m;
+    if (float_kind(L.kind)) return m > 8 && !gemm_float_supported(L, a) ? gemm_float_scratch_want(m, L.k) : 0;
+    return std::max(m > 8 && gemm_supported(L, a) ? gemm_scratch_bytes(L, m) : 0, gemv_scratch_bytes(8, L.k));
+}
+
+// An encode's scratch for its products: memory of the most any of them needs,
+// taken by the first, beside the kernels queued before it (grown product by
+// product, each growth waited for the device to free the smaller one).
+struct ProductScratch {
+    DeviceMemory& mem;
+    size_t most = 0;
+    void plan(const Layer& L, int m) { most = std::max(most, product_scratch(L, m)); }
+    void* get() {
+        if (mem.bytes < most) mem.alloc(most);
+        return mem.ptr;
+    }
+};
+
 // x W^T (+ bias) of m rows into y: then the GELU, then + residual. The
 // matrix cores for more than 8 rows, the GELU and the add in their store;
 // else launches of up to 8 rows. conv: the rows are a convolution's im2col
 // columns (ConvInput; its maps are `maps`), which take the place of x --
 // quantized from the maps where the layer allows it, else written to x.
 void encoder_product(const Layer& L, float* x, int m, float* y, const float* residual, bool gelu,
-                     DeviceMemory& scratch, hipStream_t s, const ConvInput* conv = nullptr, int maps = 0) {
+                     ProductScratch& scratch, hipStream_t s, const ConvInput* conv = nullptr, int maps = 0) {
     GemvArgs a;
     a.x = x;
     a.y = y;
@@ -321,22 +342,12 @@ void encoder_product(const Layer& L, float* x, int m, float* y, const float* res
                            conv->bins, conv->times, conv->channels, x);
         conv = nullptr;
     }
-    if (whole) {
-        const size_t need = gemm_scratch_bytes(L, m);
-        if (scratch.bytes < need) scratch.alloc(need);
-        return gemm_int(L, a, scratch.ptr, s, conv);
-    }
+    if (whole) return gemm_int(L, a, scratch.get(), s, conv);
     if (m > 8 && gemm_float_supported(L, a)) return gemm_float(L, a, s);
-    if (m > 8 && gemm_float_mfma_supported(L, a)) {
-        const size_t need = gemm_float_scratch_want(m, L.k);
-        if (scratch.bytes < need) scratch.alloc(need);
-        return gemm_float_mfma(L, a, scratch.ptr, scratch.bytes, s);
-    }
+    if (m > 8 && gemm_float_mfma_supported(L, a)) return gemm_float_mfma(L, a, scratch.get(), scratch.most, s);
     if (!float_kind(L.kind)) {
-        const size_t need = gemv_scratch_bytes(8, L.k);
-        if (scratch.bytes < need) scratch.alloc(need);
-        a.scratch = scratch.ptr;
-        a.scratch_bytes = scratch.bytes;
+        a.scratch = scratch.get();
+        a.scratch_bytes = scratch.most;
     }
     // (A GELU's residual is added after it, below.)
     a.gelu = 0;
@@ -470,7 +481,10 @@ int trit_hip_encoder_encode(const TritHipEncoder* encoder, const float* mel, flo
         DeviceMemory& kc = ws.get(8, (size_t)P * d * 4);
         DeviceMemory& vc = ws.get(9, (size_t)P * d * 4);
         DeviceMemory& st = ws.get(10, sizeof(State));
-        DeviceMemory& scratch = ws.bufs[11];
+        ProductScratch scratch{ws.bufs[11]};
+        scratch.plan(*e.conv1, frames);
+        scratch.plan(*e.conv2, P);
+        for (const LayerRef& L : e.layers) scratch.plan(*L, P);
         TRIT_HIP(hipMemcpyAsync(dmel.ptr, mel, (size_t)frames * c.mels * 4, hipMemcpyHostToDevice, s));
         State h0{};  // pos = tk - tq = 0: every query sees every key (no mask)
         TRIT_HIP(hipMemcpyAsync(st.ptr, &h0, sizeof(State), hipMemcpyHostToDevice, s));
@@ -608,7 +622,10 @@ int trit_hip_asr_encoder_encode(const TritHipAsrEncoder* encoder, const float* m
         DeviceMemory& kc = ws.get(8, (size_t)window * d * 4);
         DeviceMemory& vc = ws.get(9, (size_t)window * d * 4);
         DeviceMemory& st = ws.get(10, sizeof(State));
-        DeviceMemory& scratch = ws.bufs[11];
+        ProductScratch scratch{ws.bufs[11]};
+        for (int i = 0; i < 3; ++i) scratch.plan(*e.convs[i], maps * bins[i + 1] * times[i + 1]);
+        for (const LayerRef& L : {e.conv_out, e.proj1, e.proj2}) scratch.plan(*L, t);
+        for (const LayerRef& L : e.layers) scratch.plan(*L, t);
         TRIT_HIP(hipMemcpyAsync(dmel.ptr, mel, (size_t)frames * c.mels * 4, hipMemcpyHostToDevice, s));
         State h0{};  // pos = tk - tq = 0: every row of a window sees the whole window
         TRIT_HIP(hipMemcpyAsync(st.ptr, &h0, sizeof(State), hipMemcpyHostToDevice, s));
