@@ -1427,7 +1427,12 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_rows_kernel(
     const KV* __restrict__ vcache, int max_pos, int rows, float* __restrict__ out, const State* st, int causal) {
     if (st->done) return;
     extern __shared__ float sm[];  // qh[R][MAX_HD] | probs[R][pitch] | red[R][ATT_THREADS / 64] | inv[R]
-    const int h = blockIdx.x, row0 = blockIdx.y * R;
+    // Blocks head by head, an eighth of them on each XCD (block b runs on XCD
+    // b % 8), as the matrix-core kernel's: an XCD's L2 holds its heads' keys.
+    const int tiles = (rows + R - 1) / R, per = gridDim.x / 8;
+    const int id = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if (id >= heads * tiles) return;
+    const int h = id / tiles, row0 = (id % tiles) * R;
     const int nr = min(R, rows - row0);
     const int g = h / (heads / kvh);
     const int tk = st->pos + rows;
@@ -1612,7 +1617,7 @@ bool launch_attention_rows(const float* qkv, int stride, int heads, int kvh, int
     constexpr size_t LIMIT = 64 * 1024;
     auto go = [&](auto R_) {
         constexpr int R = decltype(R_)::value;
-        hipLaunchKernelGGL((attention_rows_kernel<KV, R>), dim3(heads, (rows + R - 1) / R), dim3(ATT_THREADS),
+        hipLaunchKernelGGL((attention_rows_kernel<KV, R>), dim3((heads * ((rows + R - 1) / R) + 7) / 8 * 8), dim3(ATT_THREADS),
                            rows_lds(R, max_tk), s, qkv, stride, heads, kvh, hd, kc, vc, max_pos, rows, out, st, causal);
         return true;
     };
