@@ -69,36 +69,6 @@ __device__ __forceinline__ void widen4(const Four<_Float16>& r, float (&f)[4]) {
     f[3] = f16_to_f32((uint16_t)(r.v.y >> 16));
 }
 
-// exp_trit (device.h) of four values at once, the same steps: a dependent
-// vector instruction costs 10.5 cycles, so four chains side by side; the
-// scheduling barriers keep the compiler from running them one after another.
-__device__ __forceinline__ void exp_trit4(float (&x)[4]) {
-    constexpr float LOG2E = 1.44269504088896340736f, LN2_HI = 0.693359375f, LN2_LO = -2.12194440e-4f;
-    float n[4], p[4], rr[4];
-    int e[4];
-#define EACH4(...)                              \
-    _Pragma("unroll") for (int i = 0; i < 4; ++i) { \
-        __VA_ARGS__;                            \
-    }                                           \
-    __builtin_amdgcn_sched_barrier(0)
-    EACH4(x[i] = __builtin_fminf(__builtin_fmaxf(x[i], -87.3f), 88.0f));
-    EACH4(n[i] = x[i] * LOG2E);
-    EACH4(n[i] = __builtin_rintf(n[i]));
-    EACH4(e[i] = (int)n[i]);
-    EACH4(n[i] = (float)e[i]);
-    EACH4(x[i] = __builtin_fmaf(-n[i], LN2_HI, x[i]));
-    EACH4(x[i] = __builtin_fmaf(-n[i], LN2_LO, x[i]));
-    EACH4(p[i] = __builtin_fmaf(1.9875691e-4f, x[i], 1.3981999e-3f));
-    EACH4(p[i] = __builtin_fmaf(p[i], x[i], 8.333452e-3f));
-    EACH4(p[i] = __builtin_fmaf(p[i], x[i], 4.1665796e-2f));
-    EACH4(p[i] = __builtin_fmaf(p[i], x[i], 0.16666665f));
-    EACH4(p[i] = __builtin_fmaf(p[i], x[i], 0.5f); rr[i] = x[i] * x[i]);
-    EACH4(x[i] = x[i] + 1.0f);
-    EACH4(p[i] = __builtin_fmaf(p[i], rr[i], x[i]));
-    EACH4(x[i] = p[i] * __builtin_bit_cast(float, (uint32_t)(e[i] + 127) << 23));
-#undef EACH4
-}
-
 template <typename KV, int VE>
 struct alignas(sizeof(KV) * VE) Values {
     KV e[VE];
@@ -246,7 +216,7 @@ __global__ __launch_bounds__(64 * W, W == 4 && (HD == 64 || sizeof(KV) == 2) ? 3
                 if (j < NT) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) s[j][r] = s[j][r] - mx;
-                    exp_trit4(s[j]);
+                    exp_trit_n<true>(s[j]);
                     buf[c & 1][(u * W + w) * WAVE + lane] = make_float4(s[j][0], s[j][1], s[j][2], s[j][3]);
                 }
             }

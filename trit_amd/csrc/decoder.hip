@@ -1598,7 +1598,11 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_rows_kernel(
 
 // Query rows from which the matrix cores take Trit's attention
 // (attention_rows.hip: tiles of 16 rows) from the vector kernel's 4 rows a
-// block.
+// block. Over f16 caches both take about the same for 9-16 rows of few keys and
+// the matrix cores are faster from there (16 heads of 128, us, vector kernel
+// and matrix cores: 9 rows over 137 keys 14.4, 15.0, over 3009 145, 124; 16 rows
+// over 144 keys 15.4, 16.1, over 1516 89, 79; 64 rows over 3064 170, 126); over f32
+// caches they are from row 9 (9 rows over 521 keys 35.5, 31.2).
 constexpr int ROWS_MFMA_MIN = 9;
 
 // Shared memory of attention_rows_kernel for R rows over tk keys.
@@ -1728,12 +1732,11 @@ void ensure_rows(SessionImpl& S, int rows) {
     S.att_arrived.alloc((size_t)rows * c.kv_heads * 4);
     const int kmax = std::max(std::max(c.d, qd), c.ffn);
     size_t scratch = std::max(gemm_scratch_bytes(rows, kmax), gemv_scratch_bytes(8, kmax));
-    // Of many rows: float-math linears' operand copy, ternary linears' padded codes.
+    // Of many rows: float-math linears' operand copy.
     const DecoderImpl& D = *S.dec;
     for (int l = 0; l < c.layers && rows > 8; ++l)
         for (const Layer* L : {D.qkv[l].get(), D.o[l].get(), D.gate_up[l].get(), D.down[l].get()})
-            scratch = std::max(scratch, float_kind(L->kind) ? gemm_float_scratch_want(rows, L->k)
-                                                            : gemm_scratch_bytes(*L, rows));
+            if (float_kind(L->kind)) scratch = std::max(scratch, gemm_float_scratch_want(rows, L->k));
     S.gemm_scratch.alloc(scratch);
     TRIT_HIP(hipMemset(S.att_arrived.ptr, 0, (size_t)rows * c.kv_heads * 4));
     S.rows_cap = rows;

@@ -31,23 +31,48 @@ __device__ __forceinline__ float f16_round(float v) { return (float)(_Float16)v;
 
 // Cephes expf with the steps of Trit's fused paths
 // (src/cpu/activation.rs:8-38,357-375; src/cpu/v2/activation.rs:45-56).
+struct ExpTrit {
+    static constexpr float LOW = -87.3f, HIGH = 88.0f, LOG2E = 1.44269504088896340736f;
+    static constexpr float LN2_HI = 0.693359375f, LN2_LO = -2.12194440e-4f;
+    static constexpr float P5 = 1.9875691e-4f, P4 = 1.3981999e-3f, P3 = 8.333452e-3f;
+    static constexpr float P2 = 4.1665796e-2f, P1 = 0.16666665f, P0 = 0.5f;
+};
+
+// exp of N values, step by step side by side. Several chains at once hide a
+// dependent vector instruction's 10.5 cycles; SIDE: scheduling barriers keep
+// the compiler from running them one after another.
+template <bool SIDE, int N>
+__device__ __forceinline__ void exp_trit_n(float (&x)[N]) {
+    using E = ExpTrit;
+    float n[N], p[N], rr[N];
+    int e[N];
+#define EACH(...)                                       \
+    _Pragma("unroll") for (int i = 0; i < N; ++i) {     \
+        __VA_ARGS__;                                    \
+    }                                                   \
+    if (SIDE) __builtin_amdgcn_sched_barrier(0)
+    EACH(x[i] = __builtin_fminf(__builtin_fmaxf(x[i], E::LOW), E::HIGH));
+    EACH(n[i] = x[i] * E::LOG2E);
+    EACH(n[i] = __builtin_rintf(n[i]));
+    EACH(e[i] = (int)n[i]);
+    EACH(n[i] = (float)e[i]);
+    EACH(x[i] = __builtin_fmaf(-n[i], E::LN2_HI, x[i]));
+    EACH(x[i] = __builtin_fmaf(-n[i], E::LN2_LO, x[i]));
+    EACH(p[i] = __builtin_fmaf(E::P5, x[i], E::P4));
+    EACH(p[i] = __builtin_fmaf(p[i], x[i], E::P3));
+    EACH(p[i] = __builtin_fmaf(p[i], x[i], E::P2));
+    EACH(p[i] = __builtin_fmaf(p[i], x[i], E::P1));
+    EACH(p[i] = __builtin_fmaf(p[i], x[i], E::P0); rr[i] = x[i] * x[i]);
+    EACH(x[i] = x[i] + 1.0f);
+    EACH(p[i] = __builtin_fmaf(p[i], rr[i], x[i]));
+    EACH(x[i] = p[i] * __builtin_bit_cast(float, (uint32_t)(e[i] + 127) << 23));
+#undef EACH
+}
+
 __device__ __forceinline__ float exp_trit(float x) {
-    constexpr float LOG2E = 1.44269504088896340736f;
-    constexpr float LN2_HI = 0.693359375f;
-    constexpr float LN2_LO = -2.12194440e-4f;
-    x = __builtin_fminf(__builtin_fmaxf(x, -87.3f), 88.0f);
-    int n_int = (int)__builtin_rintf(x * LOG2E);
-    float n = (float)n_int;
-    float r = __builtin_fmaf(-n, LN2_HI, x);
-    r = __builtin_fmaf(-n, LN2_LO, r);
-    float p = 1.9875691e-4f;
-    p = __builtin_fmaf(p, r, 1.3981999e-3f);
-    p = __builtin_fmaf(p, r, 8.333452e-3f);
-    p = __builtin_fmaf(p, r, 4.1665796e-2f);
-    p = __builtin_fmaf(p, r, 0.16666665f);
-    p = __builtin_fmaf(p, r, 0.5f);
-    float y = __builtin_fmaf(p, r * r, r + 1.0f);
-    return y * __builtin_bit_cast(float, (uint32_t)(n_int + 127) << 23);
+    float v[1] = {x};
+    exp_trit_n<false>(v);
+    return v[0];
 }
 
 // v / (1 + exp(0 - v)) (src/cpu/activation.rs:54-56,330).

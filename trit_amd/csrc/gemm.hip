@@ -19,14 +19,16 @@
 //  2. quantize_kernel: Trit's activation quantizer over all rows into codes
 //     (m x k) and group scales stored group-major (g x mpad), so that a
 //     lane's four consecutive output rows read one 16-byte load;
-//  3. gemm_kernel: 256 threads = 2 x 2 waves over 64 rows of x and 128
-//     weight rows. K runs in 256-byte chunks staged through LDS (the last
-//     one zero past k when k % 256 != 0): 16 threads
-//     read a row's 256 contiguous bytes, and the next chunk's loads are in
-//     flight while this one computes. A wave owns 32 rows of x by two
-//     32-row MFMA tiles of weights (or, for the SwiGLU pair, the gate tile
-//     and its up tile), so every (row, output) total stays in one lane's
-//     registers from the first group to the epilogue.
+//  3. the product: gemm_dma_kernel where k is a multiple of 128,
+//     gemm_ternary_kernel for ternary layers, else gemm_wide_kernel (large
+//     products) or gemm_kernel: 256 threads = 2 x 2 waves over 64 rows of x
+//     and 128 weight rows. K runs in 256-byte chunks staged through LDS (the
+//     last one zero past k): 16 threads read a row's 256 contiguous bytes,
+//     and the next chunk's loads are in flight while this one computes. A
+//     wave owns 32 rows of x by two 32-row MFMA tiles of weights (or, for
+//     the SwiGLU pair, the gate tile and its up tile), so every (row,
+//     output) total stays in one lane's registers from the first group to
+//     the epilogue.
 #include "device.h"
 #include "internal.h"
 
@@ -200,47 +202,35 @@ __global__ __launch_bounds__(256) void quantize_conv_kernel(ConvInput in, int m,
 }
 
 constexpr int KC = 256;           // bytes of K per LDS chunk
+constexpr int GPC = KC / 32;      // groups per chunk
 constexpr int ROW_LDS = KC + 16;  // padded LDS row: rows 8 apart start 4 banks apart
 constexpr int BN_ROWS = 128;      // weight rows per block
 
 // One K chunk in LDS: the block's 64 x rows and 128 weight rows, and their
 // group scales (weight scales widened to f32).
-template <int G>
 struct alignas(16) Stage {
-    static constexpr int GPC = KC / G;  // groups per chunk
     alignas(16) int8_t a[BM * ROW_LDS];
     alignas(16) int8_t b[BN_ROWS * ROW_LDS];
     alignas(16) float xs[GPC][BM];
     alignas(16) float ws[GPC][BN_ROWS];
 };
 
-// A group's operand fragments: lane (lr, h) holds bytes [16h, 16h + 16) of
-// each 32-wide step of x row lr and weight rows lr of the two tiles.
-template <int CH>
+// A group's operand fragments: lane (lr, h) holds bytes [16h, 16h + 16) of x
+// row lr and of weight rows lr of the two tiles.
 struct Frags {
-    v4i a[CH], b0[CH], b1[CH];
+    v4i a, b0, b1;
 };
 
-template <int G>
-__device__ __forceinline__ void read_frags(const int8_t* la, const int8_t* lb0, const int8_t* lb1, int gi,
-                                           Frags<G / 32>& f) {
-#pragma unroll
-    for (int s = 0; s < G / 32; ++s) {
-        const int off = gi * G + 32 * s;
-        f.a[s] = *(const v4i*)(la + off);
-        f.b0[s] = *(const v4i*)(lb0 + off);
-        f.b1[s] = *(const v4i*)(lb1 + off);
-    }
+__device__ __forceinline__ void read_frags(const int8_t* la, const int8_t* lb0, const int8_t* lb1, int gi, Frags& f) {
+    f.a = *(const v4i*)(la + 32 * gi);
+    f.b0 = *(const v4i*)(lb0 + 32 * gi);
+    f.b1 = *(const v4i*)(lb1 + 32 * gi);
 }
 
 // The i32 dots of a group for the wave's two weight tiles.
-template <int G>
-__device__ __forceinline__ void mfma_group(const Frags<G / 32>& f, v16i& d0, v16i& d1) {
-#pragma unroll
-    for (int s = 0; s < G / 32; ++s) {
-        d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[s], f.b0[s], d0, 0, 0, 0);
-        d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[s], f.b1[s], d1, 0, 0, 0);
-    }
+__device__ __forceinline__ void mfma_group(const Frags& f, v16i& d0, v16i& d1) {
+    d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a, f.b0, d0, 0, 0, 0);
+    d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a, f.b1, d1, 0, 0, 0);
 }
 
 // A group's scales for the lane: x scales of its 16 output rows (four
@@ -257,20 +247,19 @@ __device__ __forceinline__ void read_scales(const float* xs, const float* ws, in
     s.w1 = ws[c1];
 }
 
-template <int G, bool HALF, int P, bool TAIL, bool GELU>
+// Q8_0 / Q4_K products of k not a multiple of 128.
+template <int P, bool GELU>
 __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(const int8_t* __restrict__ xq,
                                                                const float* __restrict__ xs, int m, int mpad,
                                                                const int8_t* __restrict__ codes,
-                                                               const void* __restrict__ scales,
+                                                               const uint16_t* __restrict__ scales,
                                                                const float* __restrict__ bias, int n, int k,
                                                                int nb, int mb, GemvArgs a) {
-    constexpr int GPC = KC / G;  // groups per chunk
-    constexpr int CH = G / 32;   // MFMA steps per group
-    __shared__ __align__(16) Stage<G> st;
+    __shared__ __align__(16) Stage st;
     if (a.skip && *a.skip) return;
-    // TAIL: k is not a multiple of KC; the last chunk holds k % KC bytes,
-    // zero past them, and chains only its real groups.
-    const int groups = k / G, chunks = (k + KC - 1) / KC;
+    // The last chunk holds k % KC bytes, zero past them, and chains only its
+    // real groups.
+    const int groups = k / 32, chunks = (k + KC - 1) / KC;
     // Tiles in XCD order: block b runs on XCD b % 8; the blocks of one XCD
     // share weight tiles, which then stay in that XCD's L2.
     const int blk = blockIdx.x;
@@ -321,43 +310,27 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(const int8_t* __r
 
     v4i ra[4], rb[8];
     float4 rx = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    uint4 rw = make_uint4(0, 0, 0, 0);  // HALF: 8 f16 scales; else 2 f32 in .x .y
+    uint32_t rw[4] = {0, 0, 0, 0};  // 8 f16 scales
     auto fetch = [&](int c) {
         const size_t off = (size_t)c * KC;
         // Every piece of the thread sits at byte 16 (t % 16) of its row's chunk.
-        const bool in_k = !TAIL || 16 * (t % 16) < k - c * KC;
+        const bool in_k = 16 * (t % 16) < k - c * KC;
 #pragma unroll
         for (int i = 0; i < 4; ++i) ra[i] = in_k ? *(const v4i*)(xq + ag[i] + off) : v4i{0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < 8; ++i) rb[i] = in_k ? *(const v4i*)(codes + bg[i] + off) : v4i{0, 0, 0, 0};
         if (xs_thread) {
-            if (!TAIL || c * GPC + t / 16 < groups)
+            if (c * GPC + t / 16 < groups)
                 rx = *(const float4*)(xs + (size_t)(c * GPC + t / 16) * mpad + mbase + 4 * (t % 16));
             else
                 rx = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
-        if (ws_thread && TAIL) {
+        if (ws_thread) {
             // A row's scales start anywhere: one load a scale, none past the row.
-            uint32_t v[4] = {0, 0, 0, 0};
-            if (HALF) {
 #pragma unroll
-                for (int j = 0; j < GPC; ++j)
-                    if (c * GPC + j < groups)
-                        v[j / 2] |= (uint32_t)((const uint16_t*)scales)[ws_base + c * GPC + j] << (16 * (j % 2));
-            } else {
-#pragma unroll
-                for (int j = 0; j < GPC; ++j)
-                    if (c * GPC + j < groups)
-                        v[j] = __builtin_bit_cast(uint32_t, ((const float*)scales)[ws_base + c * GPC + j]);
-            }
-            rw = make_uint4(v[0], v[1], v[2], v[3]);
-        } else if (ws_thread) {
-            if (HALF) {
-                rw = *(const uint4*)((const uint16_t*)scales + ws_base + c * GPC);
-            } else {
-                const float2 f = *(const float2*)((const float*)scales + ws_base + c * GPC);
-                rw.x = __builtin_bit_cast(uint32_t, f.x);
-                rw.y = __builtin_bit_cast(uint32_t, f.y);
+            for (int j = 0; j < GPC; ++j) {
+                if (j % 2 == 0) rw[j / 2] = 0;
+                if (c * GPC + j < groups) rw[j / 2] |= (uint32_t)scales[ws_base + c * GPC + j] << (16 * (j % 2));
             }
         }
     };
@@ -374,16 +347,10 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(const int8_t* __r
         }
         if (xs_thread) *(float4*)(&st.xs[t / 16][4 * (t % 16)]) = rx;
         if (ws_thread) {
-            if (HALF) {
-                const uint32_t v[4] = {rw.x, rw.y, rw.z, rw.w};
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    st.ws[2 * j][ws_row] = f16_to_f32((uint16_t)(v[j] & 0xffff));
-                    st.ws[2 * j + 1][ws_row] = f16_to_f32((uint16_t)(v[j] >> 16));
-                }
-            } else {
-                st.ws[0][ws_row] = __builtin_bit_cast(float, rw.x);
-                st.ws[1][ws_row] = __builtin_bit_cast(float, rw.y);
+            for (int j = 0; j < 4; ++j) {
+                st.ws[2 * j][ws_row] = f16_to_f32((uint16_t)(rw[j] & 0xffff));
+                st.ws[2 * j + 1][ws_row] = f16_to_f32((uint16_t)(rw[j] >> 16));
             }
         }
     };
@@ -413,23 +380,23 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(const int8_t* __r
         // reads for group gi + 2 are in flight, and the vector ALUs run
         // group gi's f32 chain. Scheduling barriers keep the compiler from
         // folding the stages back together.
-        Frags<CH> f, fn;
+        Frags f, fn;
         v16i d0 = {}, d1 = {};
-        read_frags<G>(la, lb0, lb1, 0, f);
-        mfma_group<G>(f, d0, d1);
-        if (GPC > 1) read_frags<G>(la, lb0, lb1, 1, f);
+        read_frags(la, lb0, lb1, 0, f);
+        mfma_group(f, d0, d1);
+        read_frags(la, lb0, lb1, 1, f);
 #pragma unroll
         for (int gi = 0; gi < GPC; ++gi) {
             v16i n0 = {}, n1 = {};
-            if (gi + 1 < GPC) mfma_group<G>(f, n0, n1);
-            if (gi + 2 < GPC) read_frags<G>(la, lb0, lb1, gi + 2, fn);
+            if (gi + 1 < GPC) mfma_group(f, n0, n1);
+            if (gi + 2 < GPC) read_frags(la, lb0, lb1, gi + 2, fn);
             Scales sc;
             read_scales(st.xs[gi], st.ws[gi], xrow, sub0 + lr, sub1 + lr, sc);
             __builtin_amdgcn_sched_barrier(0);
             // Output (row 8*(r/4) + 4h + r%4, column lr) of a tile is register r.
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                if (TAIL && c * GPC + gi >= groups) break;  // past k: no chain step
+                if (c * GPC + gi >= groups) break;  // past k: no chain step
                 const float xv[4] = {sc.x[q].x, sc.x[q].y, sc.x[q].z, sc.x[q].w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
@@ -684,12 +651,6 @@ __global__ __launch_bounds__(GEMM_THREADS, TW == 2 ? 3 : 4) void gemm_dma_kernel
         }
     };
 
-    // Three stages in a ring, two in flight while one computes: a stage
-    // takes about a microsecond to arrive, longer than one stage's work.
-    // Before computing stage c a wave waits for its own loads of stage c
-    // (those of stage c + 1 may stay in flight: the wave's loads a stage
-    // are counted below), then the barrier makes every wave's loads of c
-    // visible and frees the buffer of stage c - 1 for stage c + 2.
     // Two stages: stage c + 1 loads while stage c computes. (A third stage
     // in flight, with a block fewer a CU for its LDS, measured slower.)
     auto step = [&](int c, DStage<TW>& cur, DStage<TW>& next) {
@@ -1126,9 +1087,9 @@ void launch_gemm(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStream
                      (const int8_t*)sc.xq, (const float*)sc.xs, a.m, sc.mpad, L.codes.as<int8_t>(),
                      (const void*)L.scales.ptr, L.bias.as<float>(), L.n, L.k, nb, mb, a);
     else if constexpr (G == 32)
-        launch_timed(a, gemm_kernel<G, HALF, P, true, GELU>, dim3(nb * mb), dim3(GEMM_THREADS), 0, s,
+        launch_timed(a, gemm_kernel<P, GELU>, dim3(nb * mb), dim3(GEMM_THREADS), 0, s,
                      (const int8_t*)sc.xq, (const float*)sc.xs, a.m, sc.mpad, L.codes.as<int8_t>(),
-                     (const void*)L.scales.ptr, L.bias.as<float>(), L.n, L.k, nb, mb, a);
+                     L.scales.as<uint16_t>(), L.bias.as<float>(), L.n, L.k, nb, mb, a);
     TRIT_HIP(hipGetLastError());
 }
 
