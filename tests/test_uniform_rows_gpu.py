@@ -35,24 +35,41 @@ def test_f32_keys(gpu, rows, hd):
     assert not np.isnan(want[3]).any()
 
 
-@pytest.mark.parametrize("rows", [6, 40])
-@pytest.mark.parametrize("hd", [64, 128])
-def test_f16_keys_past_their_range(gpu, rows, hd):
-    """One layer's keys of +-inf in the f16 caches; finite logits all the same."""
-    print(f"case uniform rows f16 rows={rows} hd={hd}", flush=True)
+def scaled_layer(hd, first, last):
+    """Two layers; the first one's qkv rows [first, last) 30000 times larger, so the
+    caches hold them as +-inf."""
     cfg = dict(d=256, ffn=512, layers=2, heads=4, kv_heads=2, head_dim=hd, vocab=500, eps=1e-6, rope_base=1e6,
                qk_norm=0)
     w = synth.lm_weights(cfg, config=77 + hd, sigma=0.2, norm_jitter=0.2)
     blocks = w.layers[0].qkv.reshape(-1, cfg["d"] // 32, 34).copy()
-    keys = blocks[4 * hd:6 * hd]
-    scales = keys[..., :2].copy().view(np.float16)
-    keys[..., :2] = (scales.astype(np.float32) * 30000).astype(np.float16).view(np.uint8)
+    part = blocks[first:last]
+    scales = part[..., :2].copy().view(np.float16)
+    part[..., :2] = (scales.astype(np.float32) * 30000).astype(np.float16).view(np.uint8)
     w.layers[0].qkv[...] = blocks.reshape(w.layers[0].qkv.shape)
-    ref, lm = O.Lm(cfg, w, kv_f16=True), model.build_decoder(w)
+    return cfg, O.Lm(cfg, w, kv_f16=True), model.build_decoder(w)
+
+
+@pytest.mark.parametrize("rows", [6, 40])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_f16_keys_past_their_range(gpu, rows, hd):
+    """One layer's keys of +-inf in the f16 caches; finite logits all the same."""
+    print(f"case uniform rows f16 keys rows={rows} hd={hd}", flush=True)
+    cfg, ref, lm = scaled_layer(hd, 4 * hd, 6 * hd)
     p = synth.prompt(78, rows, cfg["vocab"])
     s = lm.session(rows + 8)
     want = ref.forward(p)
     assert np.isfinite(want).all()
     assert same_or_both_nan(s.prefill(p), want)
+    s.free()
+    lm.free()
+
+
+@pytest.mark.parametrize("rows", [6, 40])
+def test_f16_values_past_their_range(gpu, rows):
+    print(f"case f16 values rows={rows}", flush=True)
+    cfg, ref, lm = scaled_layer(64, 6 * 64, 8 * 64)
+    p = synth.prompt(78, rows, cfg["vocab"])
+    s = lm.session(rows + 8)
+    assert same_or_both_nan(s.prefill(p), ref.forward(p))
     s.free()
     lm.free()

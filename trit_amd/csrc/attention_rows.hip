@@ -102,7 +102,9 @@ __global__ __launch_bounds__(64 * W, W == 4 && (HD == 64 || sizeof(KV) == 2) ? 3
     // below 7.7e-34, under half a step of any |out| >= 2^-80, and the chains
     // stop at kmax (nearer 0 they go on, below); f32 values take every key.
     // (Sums of less than 1: the row's maximum is infinite or all its scores
-    // are NaN, every key weighs the same, and sum and chains go on.)
+    // are NaN, every key weighs the same, and sum and chains go on. An
+    // infinite f16 value past kmax, which Trit's chain would carry into this
+    // row, is left out here; the forward's last row sees it in both.)
     const int kmax = a.causal ? min(tk, pos + row0 + nr) : tk;
     const int kend = sizeof(KV) == 2 ? kmax : tk;
     const int ntiles = (kend + TILE - 1) / TILE;
