@@ -53,3 +53,27 @@ def test_ternary_rows(gpu, n, k):
     finally:
         D.free()
         layer.free()
+
+
+# The tiles' rules: 32 x 64 outputs a block from 512 blocks (or a round of 224 to
+# 256 with long rows), 32 x 16 before; steps that are and are not a multiple of four.
+@pytest.mark.parametrize("kind,n,k,m", [
+    ("f16", 2049, 320, 500), ("f16", 1984, 320, 512), ("f16", 2048, 333, 510), ("f16", 512, 1040, 897),
+    ("f16", 450, 1024, 1030), ("f32", 640, 192, 1650), ("f32", 1100, 1001, 930), ("f32", 512, 1024, 1000),
+    ("q8", 2100, 288, 512), ("q8", 470, 1056, 1020)])
+def test_float_tiles(gpu, kind, n, k, m):
+    print(f"case tiles {kind} n={n} k={k} m={m}", flush=True)
+    layer, w = layer_and_weights(kind, n, k)
+    x = synth.activations(74 + m, m, k)
+    assert bits_equal(layer.forward(x), O.matmul_f32(x, w, O.isa_best()))
+    layer.free()
+
+
+@pytest.mark.parametrize("n,k,m", [(4096, 256, 320), (4096, 256, 321), (4090, 384, 340), (1500, 256, 1000)])
+def test_ternary_tiles(gpu, n, k, m):
+    print(f"case tiles ternary n={n} k={k} m={m}", flush=True)
+    codes, scales = synth.ternary_matrix(synth.seed_for(75, n), n, k)
+    layer = hip.Dense.ternary(codes, scales)
+    x = synth.activations(76 + m, m, k)
+    assert bits_equal(layer.forward(x), O.Ternary(codes, scales)(x))
+    layer.free()

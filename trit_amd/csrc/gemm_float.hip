@@ -266,8 +266,12 @@ __global__ __launch_bounds__(THREADS, 2) void float_mfma_kernel(const float4* __
     }
 }
 
-// Tiles of 32 rows x 64 columns; 32 x 16 where those would leave CUs
-// without a block (fewer than 256).
+// Tiles of 32 rows x 64 columns from 512 blocks of them, else 32 x 16: between
+// one block a CU and two, half the CUs would wait for the others' second. (A
+// whole round of long f16 or Q8 rows takes them too.) 16 columns against 64, us, by
+// the blocks of 64: f16 512x512 192 13.2, 14.7, 320 17.7, 21.9, 376 21.6, 23.8, 512
+// 27.0, 26.0, 1024 46.8, 38.9; 512x2048 256 37.6, 35.7, 376 52.7, 59.1, 512 81.8,
+// 60.8; f32 512x2048 256 38.8, 42.3, 376 53.6, 62.6, 512 82.3, 64.7.
 template <int K, bool VEC>
 void launch_tiles(const Layer& L, const GemvArgs& a, const float4* xt, hipStream_t s) {
     using E = typename WT<K>::E;
@@ -279,7 +283,9 @@ void launch_tiles(const Layer& L, const GemvArgs& a, const float4* xt, hipStream
                            dim3(nbn * nbm), dim3(THREADS), 0, s, xt, tiles, nb, L.codes.as<E>(),
                            K == WK_Q8 ? L.scales.as<float>() : nullptr, L.bias.as<float>(), L.n, L.k, nbn, nbm, a);
     };
-    if ((int64_t)((L.n + 63) / 64) * nbm >= 256) go(std::integral_constant<int, 4>{});
+    const int64_t blocks = (int64_t)((L.n + 63) / 64) * nbm;
+    const bool round = K != WK_F32 && L.k >= 1024 && blocks >= 224 && blocks <= 256;
+    if (blocks >= 512 || round) go(std::integral_constant<int, 4>{});
     else go(std::integral_constant<int, 1>{});
 }
 
