@@ -1093,8 +1093,11 @@ void launch_gemm(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStream
     TRIT_HIP(hipGetLastError());
 }
 
-// Two weight tiles a wave where that still makes a block for every CU, else
-// one.
+// Two weight tiles a wave from 192 blocks of them, else one: fewer leave CUs
+// without a block. One tile against two, us (quantizer included), by the blocks
+// of two: 1024x4096 128 28.0, 33.8, 192 39.4, 34.5, 256 41.6, 36.8; 4096x1024 64
+// 9.8, 12.5, 192 14.1, 13.7, 1024 40.9, 34.9; 2048x2048 128 15.0, 18.7, 192 22.3,
+// 20.6.
 void launch_ternary(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStream_t s) {
     const int mb = sc.mpad / BM;
     auto go = [&](auto TN_) {
@@ -1104,7 +1107,7 @@ void launch_ternary(const Layer& L, const GemvArgs& a, const Scratch& sc, hipStr
                      dim3(GEMM_THREADS), 0, s, (const int8_t*)sc.xq, (const float*)sc.xs, a.m, sc.mpad,
                      L.codes.as<uint8_t>(), L.scales.as<float>(), L.bias.as<float>(), L.n, L.k, nb, mb, a);
     };
-    if ((int64_t)((L.n + 127) / 128) * mb >= 256) go(std::integral_constant<int, 2>{});
+    if ((int64_t)((L.n + 127) / 128) * mb >= 192) go(std::integral_constant<int, 2>{});
     else go(std::integral_constant<int, 1>{});
     TRIT_HIP(hipGetLastError());
 }
