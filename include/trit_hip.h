@@ -127,7 +127,9 @@ int trit_hip_layer_f16(int n, int k, const uint16_t *weights, const float *bias,
  * f32, host memory. Replaces Dense::forward / forward_relu
  * (reference src/cpu/gemm.rs:500-542). Up to 8 rows run on the small-batch
  * GEMV kernels; more rows run on the matrix cores (int8 MFMA for the
- * integer kinds, f32 MFMA for the float-math ones), with the same bits. */
+ * integer kinds, f32 MFMA for the float-math ones; 9 to 16 ternary or
+ * float-math rows of few outputs as two launches of up to 8 where those
+ * are shorter), with the same bits. */
 int trit_hip_layer_forward(const TritHipLayer *layer, const float *x, int m, int relu, float *y);
 
 /* The same on device pointers, enqueued on `stream` (a hipStream_t; NULL:
