@@ -15,7 +15,12 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "lib", "libtrit_hip.so")
 # The measurement build: the persistent step's phase stamps compiled in.
 OUT_STAMPS = os.path.join(HERE, "lib", "libtrit_hip_stamps.so")
-SOURCES = ["layer.hip", "gemv.hip", "gemv_decode.hip", "gemv_stream.hip", "gemv_float.hip", "gemm.hip", "gemm_float.hip", "decoder.hip", "decode_step.hip", "attention_mfma.hip", "attention_rows.hip", "gguf.hip", "encoder.hip", "tokenizer.cpp"]
+SOURCES = [
+    "layer.hip", "gemv.hip", "gemv_decode.hip", "gemv_stream.hip", "gemv_float.hip", "float_rows.hip", "gemm.hip",
+    "gemm_gelu.hip", "gemm_float.hip", "decoder.hip", "decode_step.hip", "attention_mfma.hip", "attention_rows.hip",
+    "attention_rows_f16_64.hip", "attention_rows_f16_128.hip", "attention_rows_f32_64.hip",
+    "attention_rows_f32_128.hip", "gguf.hip", "encoder.hip", "tokenizer.cpp",
+]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

@@ -27,8 +27,7 @@
 // to 2048 x 512, and the stem) were bound by the launches and the vector
 // chains: 23.5 ms for its stem and two layers; here 0.49 ms, 0.08 ms of it
 // the operand copies.
-#include "device.h"
-#include "internal.h"
+#include "float_weights.h"
 
 #include <type_traits>
 
@@ -69,16 +68,6 @@ __global__ __launch_bounds__(THREADS) void chain_tile_kernel(const float* __rest
         out[(((size_t)i * nb + b) * tiles + rt) * WAVE + lane] = make_float4(p[0], p[64], p[128], p[192]);
     }
 }
-
-enum WKind { WK_F16, WK_F32, WK_Q8 };
-template <int K>
-struct WT;
-template <>
-struct WT<WK_F16> { using E = uint16_t; };
-template <>
-struct WT<WK_F32> { using E = float; };
-template <>
-struct WT<WK_Q8> { using E = int8_t; };
 
 // Four consecutive chain steps of one weight row as loaded.
 template <int K>

@@ -14,8 +14,7 @@
 // Q8 scales stay row-major [j][kk / 32] (step s of any lane is in group
 // s / 2). The tree is four cross-lane shuffles inside each 16-lane group;
 // f32 addition commutes, so both lanes of a pair hold the same bits.
-#include "device.h"
-#include "internal.h"
+#include "float_weights.h"
 
 #include <type_traits>
 
@@ -26,48 +25,12 @@ constexpr int THREADS = 256;
 constexpr int MAXF = 8;
 constexpr int ROWS = THREADS / 16;  // rows per block step
 
-// Weight kinds: element type and elements per 16-byte unit.
-enum WKind { WK_F16, WK_F32, WK_Q8 };
-template <int K>
-struct WT;
-template <>
-struct WT<WK_F16> {
-    using E = uint16_t;
-    static constexpr int PER = 8;
-};
-template <>
-struct WT<WK_F32> {
-    using E = float;
-    static constexpr int PER = 4;
-};
-template <>
-struct WT<WK_Q8> {
-    using E = int8_t;
-    static constexpr int PER = 16;
-};
-
 // Element h of a 16-byte unit as f32 (a Q8 code before its scale).
 template <int K>
 __device__ __forceinline__ float elem(const uint32_t (&words)[4], int h) {
     if constexpr (K == WK_F16) return f16_to_f32((uint16_t)(words[h >> 1] >> ((h & 1) * 16)));
     else if constexpr (K == WK_F32) return __uint_as_float(words[h]);
     else return (float)(int8_t)(uint8_t)(words[h >> 2] >> ((h & 3) * 8));
-}
-
-// One element of a chain, widened: w[s] (f16, f32) or f32(code) * scale.
-template <int K>
-__device__ __forceinline__ float widen1(const typename WT<K>::E* chain, const float* row_scales, int s) {
-    if constexpr (K == WK_F16) return f16_to_f32(chain[s]);
-    else if constexpr (K == WK_F32) return chain[s];
-    else return (float)chain[s] * row_scales[s >> 1];
-}
-
-__device__ __forceinline__ void store_out(const GemvArgs& a, const float* __restrict__ bias, int n, int f, int row,
-                                          float v) {
-    if (bias) v = v + bias[row];
-    if (a.relu) v = __builtin_fmaxf(v, 0.0f);
-    const size_t at = (size_t)f * n + row;
-    a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v : v;
 }
 
 __device__ __forceinline__ float tree16(float v) {
@@ -294,55 +257,6 @@ __global__ __launch_bounds__(THREADS) void float_chunked_kernel(const typename W
     }
 }
 
-// Many input rows of a layer with few inputs (k <= 16 S; an audio stem's
-// first convolution): block (x, y) takes 256 output columns and RB input
-// rows; a thread holds its column's 16 lane chains (S steps each) in
-// registers and runs them over the rows, then the tree16 order of the
-// small-batch kernels, so every row gets their bits.
-template <int K, int S, bool GELU>
-__global__ __launch_bounds__(THREADS) void float_rows_kernel(const typename WT<K>::E* __restrict__ w,
-                                                             const float* __restrict__ scales,
-                                                             const float* __restrict__ bias, int n, int k, GemvArgs a) {
-    constexpr int RB = 64;
-    const int col = blockIdx.x * THREADS + (int)threadIdx.x;
-    if (col >= n) return;
-    const int s_count = chain_steps(k);  // <= S
-    float wr[16][S];
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-#pragma unroll
-        for (int st = 0; st < S; ++st)
-            wr[i][st] = st < s_count ? widen1<K>(w + ((size_t)col * 16 + i) * s_count,
-                                                 scales ? scales + (size_t)col * (k / 32) : nullptr, st)
-                                     : 0.0f;
-    const int f1 = min(a.m, (int)(blockIdx.y + 1) * RB);
-    for (int f = blockIdx.y * RB; f < f1; ++f) {
-        const float* xf = a.x + (size_t)f * k;
-        float l[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            float acc = 0.0f;
-#pragma unroll
-            for (int st = 0; st < S; ++st) {
-                const int kk = 16 * st + i;
-                acc = __builtin_fmaf(kk < k ? xf[kk] : 0.0f, wr[i][st], acc);
-            }
-            l[i] = acc;
-        }
-        float h[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) h[i] = l[i] + l[i + 8];
-        float v[1] = {((h[0] + h[4]) + (h[2] + h[6])) + ((h[1] + h[5]) + (h[3] + h[7]))};
-        if constexpr (GELU) {
-            finish_outputs<true>(v, bias, {col}, a.relu);
-            const size_t at = (size_t)f * n + col;
-            a.y[at] = a.epilogue == EPI_RESIDUAL ? a.residual[at] + v[0] : v[0];
-        } else {
-            store_out(a, bias, n, f, col, v[0]);
-        }
-    }
-}
-
 // Lane-chain layout from row-major weights (the padding past k is left as
 // the caller cleared it).
 template <typename E>
@@ -426,34 +340,6 @@ void gemv_float(const Layer& L, const GemvArgs& a, hipStream_t s) {
         case F32: launch_float<WK_F32>(L, a, s); break;
         case Q8_F32: launch_float<WK_Q8>(L, a, s); break;
         default: fail("float gemv: not a float-math layer");
-    }
-    TRIT_HIP(hipGetLastError());
-}
-
-bool gemm_float_supported(const Layer& L, const GemvArgs& a) {
-    return float_kind(L.kind) && L.k <= 128 && a.m >= 1 && !a.norm_w && a.epilogue != EPI_SILU_PAIR;
-}
-
-void gemm_float(const Layer& L, const GemvArgs& a, hipStream_t s) {
-    if (!gemm_float_supported(L, a)) fail("float rows: a float-math layer of k <= 128, no prologue or pair");
-    auto go = [&](auto K_, auto S_) {
-        constexpr int K = decltype(K_)::value, S = decltype(S_)::value;
-        using E = typename WT<K>::E;
-        const dim3 grid((L.n + THREADS - 1) / THREADS, (a.m + 63) / 64);
-        launch_timed(a, a.gelu ? float_rows_kernel<K, S, true> : float_rows_kernel<K, S, false>, grid, dim3(THREADS), 0,
-                     s, L.codes.as<E>(), K == WK_Q8 ? L.scales.as<float>() : nullptr, L.bias.as<float>(), L.n, L.k, a);
-    };
-    auto by_steps = [&](auto K_) {
-        const int steps = chain_steps(L.k);
-        if (steps <= 1) go(K_, std::integral_constant<int, 1>{});
-        else if (steps <= 2) go(K_, std::integral_constant<int, 2>{});
-        else if (steps <= 4) go(K_, std::integral_constant<int, 4>{});
-        else go(K_, std::integral_constant<int, 8>{});
-    };
-    switch (L.kind) {
-        case F16: by_steps(std::integral_constant<int, WK_F16>{}); break;
-        case F32: by_steps(std::integral_constant<int, WK_F32>{}); break;
-        default: by_steps(std::integral_constant<int, WK_Q8>{}); break;
     }
     TRIT_HIP(hipGetLastError());
 }
