@@ -25,7 +25,7 @@
 // Bound: the f32 matrix rate (139 TFLOP/s in a register-only loop). In
 // launches of 8 rows Whisper base's encoder products (1500 rows, 512 x 512
 // to 2048 x 512, and the stem) were bound by the launches and the vector
-// chains: 23.5 ms for its stem and two layers; here 0.49 ms, 0.08 ms of it
+// chains: 23.5 ms for its stem and two layers; here 0.47 ms, 0.07 ms of it
 // the operand copies.
 #include "float_weights.h"
 

@@ -880,7 +880,7 @@ bool narrow(int n, int mb) {
 
 // Whether a plain product takes gemm_wide_kernel: k not a multiple of 128, and
 // more 128 x 128 blocks than gemm_kernel's, two a CU, hold at once (256: past
-// them that kernel starts a second round), or rows long enough that half the
+// them that kernel starts a second wave of blocks), or rows long enough that half the
 // loads a byte pay earlier. gemm_kernel against it, us (quantizer included): n
 // 480, 384 blocks, k 32 15.8, 13.1, k 1056 61.7, 48.9, k 4320 244, 157; 192
 // blocks, k 160 13.2, 14.7, k 1056 35.4, 35.3, k 2080 58.3, 57.1, k 4320 119,
